@@ -31,6 +31,7 @@
 // one split list per row: prefix splits, then private ones.
 // No cross-workgroup synchronisation happens inside a launch.
 #include <mutex>
+#include <type_traits>
 
 #include "kq_common.h"
 
@@ -70,6 +71,9 @@ struct SdpaArgs {
     // here from the device starts
     int32_t padded;
     int64_t pad_batch_stride, pad_head_stride;
+    // direct != 0 (padded mode): the split grid is (split, kv head, row), so a
+    // wave finds its unit without the scan over the rows' split counts
+    int32_t direct;
 };
 
 template <bool BF>
@@ -89,7 +93,7 @@ __device__ __forceinline__ uint32_t pack2(float a, float b) {
         return (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)a) |
                ((uint32_t)__builtin_bit_cast(uint16_t, (_Float16)b) << 16);
     } else {
-        return (uint32_t)kq_f32_to_bf16_bits(a) | ((uint32_t)kq_f32_to_bf16_bits(b) << 16);
+        return kq_f32x2_to_bf16_bits(a, b);
     }
 }
 
@@ -185,6 +189,18 @@ __device__ __forceinline__ bool map_unit(const SdpaArgs &a, int u, int &b, int &
     return false;
 }
 
+// Largest of v over the four lane groups (lanes r, r + 16, r + 32, r + 48), in
+// every one of them: row swaps inside the VALU, where LDS shuffles put two
+// round trips into a tile's serial chain.
+__device__ __forceinline__ float max_over_groups(float v) {
+    const uint32_t u = __builtin_bit_cast(uint32_t, v);
+    const auto a = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+    const uint32_t w = __builtin_bit_cast(
+        uint32_t, fmaxf(__builtin_bit_cast(float, (uint32_t)a[0]), __builtin_bit_cast(float, (uint32_t)a[1])));
+    const auto b = __builtin_amdgcn_permlane32_swap(w, w, false, false);
+    return fmaxf(__builtin_bit_cast(float, (uint32_t)b[0]), __builtin_bit_cast(float, (uint32_t)b[1]));
+}
+
 // Tokens per K/V tile: 32, or 16 at head dim 512, where a 32-token tile
 // alone would take 256 VGPRs.  A 16-token tile fills the first half of the
 // P.V MFMA's 32 k values; the other half gets zero P and zero V rows.
@@ -205,23 +221,32 @@ struct KVTile {
     u32x4 v[NG][VT];  // token t0 + {4g+i | 16+4g+i-4}, d = 128dg + 8r .. +7
 
     // Tokens past t_end are read from the row's last token (a valid address);
-    // their scores are masked to -inf, so they contribute p = 0.
+    // their scores are masked to -inf, so they contribute p = 0.  kp, vp, t0
+    // and t_end are uniform over the wave: the tile's first row is a scalar
+    // base and a lane's rows are 32-bit offsets from it (at head dim 512 that
+    // form spilled 12 bytes a lane in the cascade, so rows count from kp).
     __device__ __forceinline__ void load(const uint16_t *kp, const uint16_t *vp, int t0, int t_end) {
         const int lane = kq_lane();
         const int r = lane & 15, g = lane >> 4;
+        using Off = std::conditional_t<(D > 256), int64_t, uint32_t>;
+        const int first = D > 256 ? 0 : min(t0, t_end - 1);
+        const int last = t_end - 1 - first;
+        t0 -= first;
+        kp += (int64_t)first * D;
+        vp += (int64_t)first * D;
 #pragma unroll
         for (int ch = 0; ch < CH; ++ch) {
-            const int tok = min(t0 + 16 * ch + r, t_end - 1);
+            const Off tok = (Off)min(t0 + 16 * ch + r, last);
 #pragma unroll
-            for (int c = 0; c < NC; ++c) k[ch][c] = *(const u32x4 *)(kp + (int64_t)tok * D + 32 * c + 8 * g);
+            for (int c = 0; c < NC; ++c) k[ch][c] = *(const u32x4 *)(kp + (tok * D + 32 * c + 8 * g));
         }
 #pragma unroll
         for (int dg = 0; dg < NG; ++dg) {
-            const int d0 = min(128 * dg + 8 * r, D - 8);
+            const uint32_t d0 = min(128 * dg + 8 * r, D - 8);
 #pragma unroll
             for (int i = 0; i < VT; ++i) {
-                const int tok = min(t0 + (i < 4 ? 4 * g + i : 16 + 4 * g + (i - 4)), t_end - 1);
-                v[dg][i] = *(const u32x4 *)(vp + (int64_t)tok * D + d0);
+                const Off tok = (Off)min(t0 + (i < 4 ? 4 * g + i : 16 + 4 * g + (i - 4)), last);
+                v[dg][i] = *(const u32x4 *)(vp + (tok * D + d0));
             }
         }
     }
@@ -257,13 +282,10 @@ __device__ __forceinline__ u32x4 deq8(u32x2 q, uint32_t sb) {
         return u32x4{pair(q.x, KQ_SEL_B01), pair(q.x, KQ_SEL_B23), pair(q.y, KQ_SEL_B01), pair(q.y, KQ_SEL_B23)};
     } else {
         const float s = f16bits_to_f32<BF>(sb & 0xFFFFu), b = f16bits_to_f32<BF>(sb >> 16);
-        float f[8];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            f[j] = fmaf((float)((q.x >> (8 * j)) & 0xFFu), s, b);
-            f[4 + j] = fmaf((float)((q.y >> (8 * j)) & 0xFFu), s, b);
-        }
-        return u32x4{pack2<BF>(f[0], f[1]), pack2<BF>(f[2], f[3]), pack2<BF>(f[4], f[5]), pack2<BF>(f[6], f[7])};
+        auto pair = [&](uint32_t w, int j) {
+            return pack2<BF>(fmaf((float)((w >> (8 * j)) & 0xFFu), s, b), fmaf((float)((w >> (8 * j + 8)) & 0xFFu), s, b));
+        };
+        return u32x4{pair(q.x, 0), pair(q.x, 2), pair(q.y, 0), pair(q.y, 2)};
     }
 }
 
@@ -306,36 +328,43 @@ struct KVTileQ8 {
                                          const uint16_t *vs, const uint16_t *vb, int t0, int t_end) {
         const int lane = kq_lane();
         const int r = lane & 15, g = lane >> 4;
-        tlast = max(t_end - 1 - t0, 0);  // (a prefetched tile past the end: every token is the last)
+        const int first = min(t0, t_end - 1);
+        const uint32_t last = (uint32_t)(t_end - 1 - first);
+        tlast = (int)last;  // (a prefetched tile past the end: every token is the last)
+        kp += (int64_t)first * D;
+        vp += (int64_t)first * D;
+        ks += (int64_t)first * SG;
+        kb += (int64_t)first * SG;
+        vs += (int64_t)first * SG;
+        vb += (int64_t)first * SG;
 #pragma unroll
         for (int ch = 0; ch < CH; ++ch) {
-            const int tok = min(t0 + 16 * ch + r, t_end - 1);
+            const uint32_t tok = min((uint32_t)(16 * ch + r), last);
             if constexpr (WK) {
 #pragma unroll
                 for (int i = 0; i < NC / 2; ++i) {
-                    const u32x4 w = *(const u32x4 *)(kp + (int64_t)tok * D + 64 * i + 16 * g);
+                    const u32x4 w = *(const u32x4 *)(kp + (tok * D + 64 * i + 16 * g));
                     k[ch][2 * i] = u32x2{w.x, w.y};
                     k[ch][2 * i + 1] = u32x2{w.z, w.w};
                 }
             } else {
 #pragma unroll
-                for (int c = 0; c < NC; ++c) k[ch][c] = *(const u32x2 *)(kp + (int64_t)tok * D + qk_d<WK>(c, g));
+                for (int c = 0; c < NC; ++c) k[ch][c] = *(const u32x2 *)(kp + (tok * D + (uint32_t)qk_d<WK>(c, g)));
             }
         }
 #pragma unroll
         for (int dg = 0; dg < NG; ++dg) {
-            const int d0 = min(128 * dg + 8 * r, D - 8);
+            const uint32_t d0 = min(128 * dg + 8 * r, D - 8);
 #pragma unroll
             for (int i = 0; i < VT; ++i) {
-                const int tok = min(t0 + (i < 4 ? 4 * g + i : 16 + 4 * g + (i - 4)), t_end - 1);
-                v[dg][i] = *(const u32x2 *)(vp + (int64_t)tok * D + d0);
+                const uint32_t tok = min((uint32_t)(i < 4 ? 4 * g + i : 16 + 4 * g + (i - 4)), last);
+                v[dg][i] = *(const u32x2 *)(vp + (tok * D + d0));
             }
         }
 #pragma unroll
         for (int j = 0; j < PJ; ++j) {
-            const int p = min(64 * j + lane, NP - 1);  // (lanes past the pairs repeat the last)
-            const int tok = min(t0 + p % TT, t_end - 1);
-            const int64_t si = (int64_t)tok * SG + p / TT;
+            const uint32_t p = min(64 * j + lane, NP - 1);  // (lanes past the pairs repeat the last)
+            const uint32_t si = min(p % TT, last) * SG + p / TT;
             ksb[j] = (uint32_t)ks[si] | ((uint32_t)kb[si] << 16);
             vsb[j] = (uint32_t)vs[si] | ((uint32_t)vb[si] << 16);
         }
@@ -427,20 +456,35 @@ struct SplitState {
         float tmax = sv[0];
 #pragma unroll
         for (int i = 1; i < 8; ++i) tmax = fmaxf(tmax, sv[i]);
-        tmax = fmaxf(tmax, __shfl_xor(tmax, 16));
-        tmax = fmaxf(tmax, __shfl_xor(tmax, 32));
+        tmax = max_over_groups(tmax);
         const float m_new = fmaxf(m_run, tmax);
-        // m_new == -inf only for heads >= G
-        const float alpha = (m_new == -INFINITY) ? 1.f : exp2f(m_run - m_new);
+        // m_new == -inf only for heads >= G.  Every argument is <= 0 and the
+        // powers are summed with 1 (the row's maximum), so the hardware's
+        // flush of results below 2^-126 is far below their rounding.
+        const bool idle = m_new == -INFINITY;
+        const float alpha = idle ? 1.f : __builtin_amdgcn_exp2f(m_run - m_new);
         float p[8];
         float psum = 0.f;
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
-            p[i] = (m_new == -INFINITY) ? 0.f : exp2f(sv[i] - m_new);
+            p[i] = idle ? 0.f : __builtin_amdgcn_exp2f(sv[i] - m_new);
             psum += p[i];
         }
         l_part = l_part * alpha + psum;
         m_run = m_new;
+        // a tile that raises no head's maximum leaves the sums as they are
+        // (alpha is exactly 1): after the first tiles most do not.  At head
+        // dim 512 the branch's copies of the sums spilled 20-56 bytes a lane,
+        // so there each sum is rescaled at its MFMA.
+        constexpr bool kSkip = NG <= 2;
+        if constexpr (kSkip) {
+            if (__builtin_amdgcn_ballot_w64(alpha != 1.f)) {
+#pragma unroll
+                for (int dg = 0; dg < NG; ++dg)
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) o[dg][j] = o[dg][j] * alpha;
+            }
+        }
         const half8_t pf = __builtin_bit_cast(
             half8_t, u32x4{pack2<BF>(p[0], p[1]), pack2<BF>(p[2], p[3]), pack2<BF>(p[4], p[5]),
                            pack2<BF>(p[6], p[7])});
@@ -457,8 +501,7 @@ struct SplitState {
                 f.y = __builtin_amdgcn_perm(vr[3][j >> 1], vr[2][j >> 1], sel);
                 f.z = __builtin_amdgcn_perm(vr[5][j >> 1], vr[4][j >> 1], sel);
                 f.w = __builtin_amdgcn_perm(vr[7][j >> 1], vr[6][j >> 1], sel);
-                const floatx4 acc = o[dg][j] * alpha;
-                o[dg][j] = mfma<BF>(__builtin_bit_cast(half8_t, f), pf, acc);
+                o[dg][j] = mfma<BF>(__builtin_bit_cast(half8_t, f), pf, kSkip ? o[dg][j] : o[dg][j] * alpha);
                 if constexpr (QL) __builtin_amdgcn_sched_barrier(0);  // (see q_lds_pitch)
             }
         }
@@ -481,10 +524,17 @@ struct KvSrc {
     const uint16_t *ks, *kb, *vs, *vb;
 };
 
+// A wave-uniform value the compiler cannot prove uniform, in scalar registers.
+__device__ __forceinline__ int64_t uniform64(int64_t v) {
+    return (int64_t)(((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(v >> 32)) << 32) |
+                     (uint32_t)__builtin_amdgcn_readfirstlane((int)v));
+}
+
 template <bool Q8>
 __device__ __forceinline__ KvSrc kv_src(const void *k, const void *v, const uint16_t *ks, const uint16_t *kb,
                                         const uint16_t *vs, const uint16_t *vb, int64_t base) {
     KvSrc r;
+    base = uniform64(base);  // one unit per wave
     if constexpr (Q8) {
         r.k = (const uint8_t *)k + base;
         r.v = (const uint8_t *)v + base;
@@ -531,6 +581,8 @@ __device__ __forceinline__ void split_unit(const SdpaArgs &a, const KvSrc &src, 
     using Tile = typename TileOf<D, BF, Q8, WK>::type;
     const int lane = kq_lane();
     const int g = lane >> 4;
+    t_begin = __builtin_amdgcn_readfirstlane(t_begin);
+    t_end = __builtin_amdgcn_readfirstlane(t_end);
 
     SplitState<D, BF, QL> st[NRB];
 #pragma unroll
@@ -639,24 +691,32 @@ __device__ __forceinline__ void split_unit(const SdpaArgs &a, const KvSrc &src, 
 // Ragged mode: unit = one wave = (row b, kv head h, split s), the G q heads
 // of the group in columns 0..G-1.
 //
-// Register budget: left alone the compiler gives a wave ~290 of the SIMD's
-// 512 registers (one wave per SIMD).  A 16-bit wave keeps one 16 KB tile in
-// flight, enough for the four waves of a CU to stream at HBM rate (C3: 0.71
-// of 8 TB/s); an 8-bit tile is half the bytes, and at one wave per SIMD the
-// 8-bit C3 batch ran at 4.2-4.3 TB/s.  8-bit kernels at head dim <= 128
-// therefore ask for two waves per SIMD (249 VGPRs, no AGPRs, no scratch):
-// 0.250 -> 0.224-0.229 ms on C3 (measured).  Three waves spill 416 B per
-// lane; two waves with a three-tile ring spill 88 B; the 16-bit kernel at two
-// waves measured the same as at one.
+// Register budget: two waves per SIMD at head dims up to 128 (at most 251
+// VGPRs, no AGPRs, no scratch), so one wave's start and end (its query and
+// first tile, its partial) run under another's tiles.  Left alone the compiler
+// takes ~290 registers, one wave: 16-bit calls at T = 16 k .. 528 k head-tokens
+// then take 3-10 % longer at 512-token splits (20.2 against 18.7 us at 36 k)
+// and the same on the C3 batch, whose waves stream at HBM rate either way; the
+// 8-bit C3 batch, with half the bytes in flight a wave, 0.250 against
+// 0.224-0.229 ms.  Three waves spill 416 B per lane, two with a three-tile
+// ring 88 B.
 template <int D, bool BF, int NBUF, bool Q8>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(Q8 && D <= 128 ? 2 : 1))) void kq_sdpa_split_kernel(
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(D <= 128 ? 2 : 1))) void kq_sdpa_split_kernel(
     SdpaArgs a) {
     __shared__ __attribute__((aligned(16))) uint8_t qs[q_in_lds<D, Q8>() ? q_lds_bytes<D>() : 16];
     const uint32_t q_lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void *)qs;
     const int r = kq_lane() & 15;
     for (int u = blockIdx.x;; u += gridDim.x) {
         int b, h, s;
-        if (!map_unit(a, u, b, h, s)) return;
+        if (a.direct) {
+            // grid (split, kv head, row): one unit per workgroup
+            s = u;
+            h = blockIdx.y;
+            b = blockIdx.z;
+            if (s >= row_unit_splits(a, b)) return;
+        } else if (!map_unit(a, u, b, h, s)) {
+            return;
+        }
         const int len = ragged_len(a, b);
         const int t_begin = s * a.split;
         const int t_end = min(len, t_begin + a.split);
@@ -665,6 +725,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(Q8 && D <= 1
         const bool ok[1] = {r < a.G};
         split_unit<D, BF, NBUF, 1, Q8>(a, kv_src<Q8>(a.k, a.v, a.ks, a.kb, a.vs, a.vb, kvbase), t_begin, t_end, h, s,
                                        rw, hd, ok, q_lds);
+        if (a.direct) return;
     }
 }
 
@@ -756,6 +817,17 @@ __global__ __launch_bounds__(256) void kq_sdpa_merge_kernel(SdpaArgs a) {
     // common max over the splits
     float M = -INFINITY;
     for (int s = t; s < nsplit; s += 256) M = fmaxf(M, ml[s * ml_stride]);
+    // this thread's first splits, in flight beside the maximum's loads
+    constexpr int PRE = 4;
+    float4 o_pre[PRE];
+    float m_pre[PRE], l_pre[PRE];
+#pragma unroll
+    for (int i = 0; i < PRE; ++i) {
+        const int s = min(part + i * P, nsplit - 1);
+        m_pre[i] = ml[s * ml_stride];
+        l_pre[i] = ml[s * ml_stride + 1];
+        o_pre[i] = po[s * po_stride];
+    }
     for (int off = 32; off > 0; off >>= 1) M = fmaxf(M, __shfl_xor(M, off));
     if ((t & 63) == 0) red_m[t >> 6] = M;
     __syncthreads();
@@ -764,17 +836,20 @@ __global__ __launch_bounds__(256) void kq_sdpa_merge_kernel(SdpaArgs a) {
     if (part < P) {
         float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
         float L = 0.f;
-#pragma unroll 4
-        for (int s = part; s < nsplit; s += P) {
-            const float ms = ml[s * ml_stride], ls = ml[s * ml_stride + 1];
-            const float f = (ms == -INFINITY) ? 0.f : exp2f(ms - M);
-            const float4 o = po[s * po_stride];
+        auto add = [&](float ms, float ls, const float4 &o) {
+            const float f = (ms == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(ms - M);
             L += ls * f;
             acc.x += f * o.x;
             acc.y += f * o.y;
             acc.z += f * o.z;
             acc.w += f * o.w;
-        }
+        };
+#pragma unroll
+        for (int i = 0; i < PRE; ++i)
+            if (part + i * P < nsplit) add(m_pre[i], l_pre[i], o_pre[i]);
+#pragma unroll 4
+        for (int s = part + PRE * P; s < nsplit; s += P)
+            add(ml[s * ml_stride], ml[s * ml_stride + 1], po[s * po_stride]);
         red_acc[part][q] = acc;
         if (q == 0) red_l[part] = L;
     }
@@ -806,16 +881,39 @@ int env_int(const char *name, int dflt) {
     return (end && *end == 0 && v > 0 && v < (1 << 24)) ? (int)v : dflt;
 }
 
-// Tokens per split (a multiple of the 32-token tile): 1024 when the launch's
-// unit bound B * Hkv * ceil(max_len / 1024) gives every CU 8 waves, 512
-// otherwise (longer splits halve the partials and the merge's work; measured
-// on C3: 353 against 372 us); GMLX_KQ_SDPA_SPLIT forces it.  The workspace
-// size follows the same rule from the same arguments.
-int split_tokens(int B, int Hkv, int max_len) {
+// Tokens per split (a multiple of the 32-token tile), by the launch's size in
+// head-tokens T = B * Hkv * max_len (max_len bounds every row).  A split is
+// one wave's chain of tiles, 0.5-0.8 us each, and one fp32 partial to write
+// and merge: short launches want short chains, long ones few partials.
+// Measured per call, D = 128 (us at 64 / 128 / 256 / 512 / 1024 tokens),
+// 16-bit:
+//   T    16 k   9.2 / 10.3 / 12.8 / 18.0 / 28.1
+//   T    36 k   11.4 / 11.5 / 13.4 / 18.7 / 28.7
+//   T   118 k   24.7 / 22.6 / 20.6 / 21.5 / 29.8
+//   T   256 k   37.3 / 32.9 / 31.5 / 30.5 / 32.1
+//   T 1 024 k   119.4 / 115.1 / 109.4 / 102.7 / 98.9
+// and over an 8-bit cache with bf16 queries
+//   T    36 k   11.9 / 14.1 / 19.1 / 29.7 / 51.2
+//   T   256 k   31.0 / 24.6 / 23.1 / 32.5 / 53.0
+//   T   528 k   53.3 / 47.5 / 46.9 / 45.7 / 55.7
+// So: 64 tokens up to seven waves a CU at that length, given that the
+// partials stay under 16 MB (wide head groups at D = 512 would not); then
+// 512, or 256 for an 8-bit cache up to 2048 waves of that length with the
+// same bound; 1024 once B * Hkv * ceil(max_len / 1024) gives every CU 8
+// waves.  `wide` keeps to 512 and 1024: the plan of a call whose workspace
+// is too small for the short splits' partials.  GMLX_KQ_SDPA_SPLIT forces
+// one length.  The workspace size follows the same rule from the same
+// arguments.
+int split_tokens(int B, int Hq, int Hkv, int D, int max_len, bool q8, bool wide) {
     int c = env_int("GMLX_KQ_SDPA_SPLIT", 0);
     if (c == 0) {
-        const int64_t units = (int64_t)B * Hkv * (((int64_t)(max_len > 0 ? max_len : 1) + 1023) / 1024);
-        c = units >= 8 * (int64_t)device_cus() ? 1024 : 512;
+        const int64_t group_bytes = (int64_t)(Hq / Hkv) * D * 4;
+        const int64_t heads = (int64_t)B * Hkv, len = max_len > 0 ? max_len : 1, cus = device_cus();
+        const auto units = [&](int64_t tokens) { return heads * ((len + tokens - 1) / tokens); };
+        if (units(1024) >= 8 * cus) c = 1024;
+        else if (wide) c = 512;
+        else if (heads * len <= 7 * 64 * cus && units(64) * group_bytes <= (int64_t)16 << 20) c = 64;
+        else c = q8 && units(256) <= 8 * cus && units(256) * group_bytes <= (int64_t)16 << 20 ? 256 : 512;
     }
     c = (c + 31) / 32 * 32;
     return c < 32 ? 32 : c;
@@ -823,16 +921,23 @@ int split_tokens(int B, int Hkv, int max_len) {
 
 struct WsLayout {
     size_t part_bytes, ml_bytes;
+    int split;
 };
 
-WsLayout ws_layout(int B, int Hq, int Hkv, int D, int max_len) {
+WsLayout ws_layout(int B, int Hq, int Hkv, int D, int max_len, bool q8, bool wide = false) {
     const int G = Hq / Hkv;
-    const int C = split_tokens(B, Hkv, max_len);
+    const int C = split_tokens(B, Hq, Hkv, D, max_len, q8, wide);
     const int64_t ms = max_len <= 0 ? 1 : (max_len + C - 1) / C;
     WsLayout w;
+    w.split = C;
     w.part_bytes = (((size_t)B * Hkv * ms * G * D * 4) + 255) & ~(size_t)255;
     w.ml_bytes = (size_t)B * Hkv * ms * G * 2 * 4;
     return w;
+}
+
+size_t ws_bytes(int B, int Hq, int Hkv, int D, int max_len, bool q8) {
+    const WsLayout w = ws_layout(B, Hq, Hkv, D, max_len, q8);
+    return w.part_bytes + w.ml_bytes;
 }
 
 // Row blocks per prefix wave: 2 (GMLX_KQ_CASCADE_NRB=1 selects one).  Four
@@ -856,7 +961,8 @@ void launch_n(const SdpaArgs &a, int grid, int block, bool merge, hipStream_t s)
             break;
         }
     } else
-        hipLaunchKernelGGL((kq_sdpa_split_kernel<D, BF, NBUF, Q8>), dim3(grid), dim3(64), 0, s, a);
+        hipLaunchKernelGGL((kq_sdpa_split_kernel<D, BF, NBUF, Q8>),
+                           a.direct ? dim3(a.max_splits, a.Hkv, a.B) : dim3(grid), dim3(64), 0, s, a);
     if (merge) hipLaunchKernelGGL((kq_sdpa_merge_kernel<D, BF>), dim3(a.B * a.Hq), dim3(256), 0, s, a);
 }
 
@@ -879,8 +985,9 @@ extern "C" {
 
 size_t kq_sdpa_workspace_bytes(int32_t B, int32_t Hq, int32_t Hkv, int32_t D, int32_t max_len) {
     if (B <= 0 || Hkv <= 0 || Hq <= 0 || Hq % Hkv || D <= 0) return 0;
-    const WsLayout w = ws_layout(B, Hq, Hkv, D, max_len);
-    return w.part_bytes + w.ml_bytes;
+    // one sizer for both caches: the larger of their plans
+    const size_t a = ws_bytes(B, Hq, Hkv, D, max_len, false), b = ws_bytes(B, Hq, Hkv, D, max_len, true);
+    return a > b ? a : b;
 }
 
 }  // extern "C"
@@ -941,9 +1048,9 @@ int ragged_impl(const void *q, const void *k, const void *v, const Q8Scales *q8,
     const uintptr_t kv_align = q8 ? 7 : 15;
     if (((uintptr_t)q & 15) || ((uintptr_t)k & kv_align) || ((uintptr_t)v & kv_align) || ((uintptr_t)out & 15))
         return KQ_ERR_BAD_ALIGN;
-    const size_t need = kq_sdpa_workspace_bytes(B, Hq, Hkv, D, max_len);
-    if (!workspace || workspace_bytes < need) return KQ_ERR_WORKSPACE_TOO_SMALL;
-    const WsLayout w = ws_layout(B, Hq, Hkv, D, max_len);
+    WsLayout w = ws_layout(B, Hq, Hkv, D, max_len, q8 != nullptr);
+    if (workspace_bytes < w.part_bytes + w.ml_bytes) w = ws_layout(B, Hq, Hkv, D, max_len, q8 != nullptr, true);
+    if (!workspace || workspace_bytes < w.part_bytes + w.ml_bytes) return KQ_ERR_WORKSPACE_TOO_SMALL;
     SdpaArgs a;
     a.q = (const uint16_t *)q;
     a.k = (const uint16_t *)k;
@@ -967,7 +1074,7 @@ int ragged_impl(const void *q, const void *k, const void *v, const Q8Scales *q8,
     a.Hq = Hq;
     a.Hkv = Hkv;
     a.G = Hq / Hkv;
-    a.split = split_tokens(B, Hkv, max_len);
+    a.split = w.split;
     a.max_splits = max_len <= 0 ? 1 : (max_len + a.split - 1) / a.split;
     a.max_len = max_len;
     a.scale_log2 = scale * 1.4426950408889634f;
@@ -975,6 +1082,7 @@ int ragged_impl(const void *q, const void *k, const void *v, const Q8Scales *q8,
     // (rows are shorter on the device side), extra waves exit at once
     const int64_t upper = (int64_t)B * Hkv * a.max_splits;
     const int grid = (int)(upper < (1 << 22) ? upper : (1 << 22));
+    a.direct = pad && upper < (1 << 22) && Hkv < (1 << 16) && B < (1 << 16);
     const bool merge = a.max_splits > 1;
     hipStream_t s = (hipStream_t)stream;
     const bool bf = dtype == KQ_DTYPE_BF16;
@@ -1127,6 +1235,7 @@ int cascade_impl(const void *q, const void *k_shared, const void *v_shared, cons
     a.priv_batch_stride = priv_batch_stride;
     a.priv_head_stride = priv_head_stride;
     a.cascade = 1;
+    a.direct = 0;
     a.padded = 0;
     a.pad_batch_stride = a.pad_head_stride = 0;
     set_q8(a, q8s, q8p);
@@ -1246,7 +1355,7 @@ extern "C" int kq_sdpa_decode_gqa_noalloc(const void *q, const void *k, const vo
                                           kq_stream_t stream) {
     if (B == 0) return KQ_OK;
     if (B < 0 || Hq <= 0 || Hkv <= 0 || Hq % Hkv || D <= 0 || L < 0) return KQ_ERR_BAD_SHAPE;
-    const size_t need = kq_sdpa_workspace_bytes(B, Hq, Hkv, D, L);
+    const size_t need = ws_bytes(B, Hq, Hkv, D, L, false);
     if (need > KQ_SDPA_NOALLOC_SCRATCH_BYTES) return KQ_ERR_WORKSPACE_TOO_SMALL;
     void *ws = nullptr;
     if (const int rc = scratch_ptr(&ws)) return rc;
