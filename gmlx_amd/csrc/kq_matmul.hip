@@ -14,6 +14,7 @@
 // chunks use 4 waves with more m-tiles each.
 #include <stdlib.h>
 
+#include "kq_gemm.h"
 #include "kq_mma.h"
 
 // kq_mv.hip: LDS-staged small-batch launch (problems validated, all live,
@@ -1034,6 +1035,39 @@ int gather_common(const void *x, int x_dtype, int64_t x_row_stride, int32_t x_pa
         x_row_stride = K;
         x_dtype = KQ_DTYPE_F16;
     }
+    // long segments: the matrix-core tiles
+    const int32_t x_rows = gather_x_rows(n_pairs, x_pair_div, x_skip);
+    if (kq_gemm_gather_eligible(n_pairs, n_experts, x_rows, x_row_stride)) {
+        KqGemmGather g;
+        g.x = (const char *)x;
+        g.x_exp = x_exp;
+        g.w0 = (const uint8_t *)w0;
+        g.w1 = (const uint8_t *)w1;
+        g.y = y;
+        g.seg_info = seg_info;
+        g.pair_order = pair_order;
+        g.b0 = ep->bias0;
+        g.b1 = w1 ? ep->bias1 : nullptr;
+        g.w_expert_bytes = w_expert_bytes;
+        g.w_row_bytes = w_row_bytes;
+        g.y_stride = y_row_stride;
+        g.b_stride = ep->bias_expert_stride;
+        g.x_row_bytes = (uint32_t)x_row_stride * 2;
+        g.x_bytes = (uint32_t)(((int64_t)(x_rows - 1) * x_row_stride + K) * 2);
+        g.x_pair_div = x_pair_div;
+        g.x_skip = x_skip;
+        g.y_skip = y_skip;
+        g.N = N;
+        g.K = K;
+        g.codec = codec;
+        g.n_pairs = n_pairs;
+        g.n_experts = n_experts;
+        g.y_dtype = y_dtype;
+        g.act = w1 ? ep->act : KQ_ACT_SILU;
+        g.limit = ep->limit;
+        g.alpha = ep->alpha;
+        return kq_gemm_gather_launch(g, s);
+    }
     // the streaming gather: weight tiles by row-contiguous direct-to-LDS
     // copies, one persistent workgroup per CU
     if (kq_sgather_eligible(codec, w1 != nullptr, N, K, w_row_bytes, n_experts))
@@ -1097,7 +1131,8 @@ size_t split_bytes(const kq_matmul_problem *problems, int n_problems) {
         if (problems[i].M > 0 && problems[i].N > 0) all[na++] = problems[i];
     if (na == 0) return 0;
     const size_t a = kq_stream_part_bytes(all, na, kq_stream_split_want(all, na)), b = kq_mms_part_bytes(all, na);
-    return a > b ? a : b;
+    const size_t c = kq_gemm_part_bytes(all, na);
+    return a > b ? (a > c ? a : c) : (b > c ? b : c);
 }
 
 }  // namespace
@@ -1257,6 +1292,24 @@ int kq_quantized_matmul_grouped(const kq_matmul_problem *problems, int n_problem
         if (env_int_flag("GMLX_KQ_MM", 1) && kq_mm_eligible(all, na, x_dtype))
             return kq_mm_launch(all, na, xe0, y_dtype, (hipStream_t)stream);
     }
+    // more than 64 rows in every problem: the matrix-core tiles, in K slices
+    // given room for their partial tiles (GMLX_KQ_GEMM=0: the dense kernel)
+    if (live > 0) {
+        kq_matmul_problem all[KQ_MAX_GROUP];
+        const int32_t *xe[KQ_MAX_GROUP];
+        int na = 0;
+        for (int i = 0; i < n_problems; ++i)
+            if (problems[i].M != 0 && problems[i].N != 0) {
+                xe[na] = exps[i];
+                all[na++] = problems[i];
+            }
+        if (kq_gemm_eligible(all, na)) {
+            const size_t pb = kq_gemm_part_bytes(all, na);
+            const bool room = pb && workspace && !((uintptr_t)workspace & 255) && workspace_bytes >= used + pb;
+            return kq_gemm_launch(all, xe, na, y_dtype, room ? (uint32_t *)workspace : nullptr,
+                                  room ? (float *)((char *)workspace + used) : nullptr, (hipStream_t)stream);
+        }
+    }
     DenseArgs a;
     int units = 0, max_chunks = 0, np = 0;
     const int mt = group_mt(problems, n_problems);
@@ -1291,6 +1344,33 @@ int kq_quantized_matmul_grouped(const kq_matmul_problem *problems, int n_problem
     else if (mt == 2) launch_dense_nw<2, 0>(nw, a, units, max_chunks, s);
     else launch_dense_nw<4, 0>(nw, a, units, max_chunks, s);
     return hipGetLastError() == hipSuccess ? KQ_OK : KQ_ERR_LAUNCH_FAILED;
+}
+
+size_t kq_glu_matmul_workspace_bytes(int32_t M, int32_t K, int x_dtype) {
+    if (M <= 0 || K <= 0 || x_dtype == KQ_DTYPE_F16) return 0;
+    return KQ_MATMUL_COUNTER_BYTES + kq_prepared_bytes(M, K);
+}
+
+int kq_glu_matmul(const void *x, int x_dtype, int64_t x_row_stride, int32_t M, int32_t K, const void *w_gate,
+                  const void *w_up, int64_t w_row_bytes, int codec, int32_t I, int act, void *h, int h_dtype,
+                  int64_t h_row_stride, void *workspace, size_t workspace_bytes, kq_stream_t stream) {
+    if (x_dtype != KQ_DTYPE_F16 && x_dtype != KQ_DTYPE_BF16 && x_dtype != KQ_DTYPE_F32) return KQ_ERR_UNSUPPORTED_DTYPE;
+    if (h_dtype != KQ_DTYPE_F32 && h_dtype != KQ_DTYPE_F16 && h_dtype != KQ_DTYPE_BF16) return KQ_ERR_UNSUPPORTED_DTYPE;
+    if (act != KQ_ACT_SILU && act != KQ_ACT_GELU) return KQ_ERR_BAD_ARGUMENT;
+    kq_matmul_problem gate{w_gate, w_row_bytes, x, x_row_stride, h, h_row_stride, M, I, K, codec}, up = gate;
+    up.w = w_up;
+    if (const int rc = validate_problem(gate)) return rc;
+    if (const int rc = validate_problem(up)) return rc;
+    const int32_t *x_exp = nullptr;
+    if (x_dtype != KQ_DTYPE_F16) gate.x_row_stride = K;  // (of the prepared rows)
+    if (I == 0 || !kq_gemm_glu_eligible(gate)) return KQ_ERR_BAD_SHAPE;
+    if (x_dtype != KQ_DTYPE_F16) {
+        if (!workspace || workspace_bytes < kq_glu_matmul_workspace_bytes(M, K, x_dtype)) return KQ_ERR_WORKSPACE_TOO_SMALL;
+        if (const int rc = kq_prepare_rows(x, x_dtype, x_row_stride, M, K, (char *)workspace + KQ_MATMUL_COUNTER_BYTES,
+                                           &x_exp, &gate.x, (hipStream_t)stream))
+            return rc;
+    }
+    return kq_gemm_glu_launch(gate, w_up, x_exp, act, h_dtype, (hipStream_t)stream);
 }
 
 size_t kq_fused_mlp_workspace_bytes(int32_t M, int32_t K, int32_t I, int32_t N, int x_dtype) {

@@ -243,7 +243,7 @@ def fused_mlp(x, gate_w, up_w, down_w, codec="q4_k", down_codec=None, act="silu"
     (default `codec`).  fp16 activations of at most 8 rows with the served
     codecs and shapes (kq_fused_mlp) run in one launch; otherwise the same
     three steps run as the reference runs them: the grouped gate|up matmul,
-    the GLU, the down matmul.""" 
+    the GLU, the down matmul (the first two as one launch past 64 rows).""" 
     _fault("fused_mlp")
     _require_gpu(x, gate_w, up_w, down_w)
     down_codec = down_codec or codec
@@ -272,13 +272,35 @@ def fused_mlp(x, gate_w, up_w, down_w, codec="q4_k", down_codec=None, act="silu"
     if rc == KQ_OK:
         _COUNTS["fused_mlp_launches"] += 1
     elif rc == _lib.KQ_ERR_BAD_SHAPE:
-        g, u = quantized_matmul_grouped([(x2, gate_w, codec), (x2, up_w, codec)], out_dtype=torch.float32)
-        gf = torch.nn.functional.silu(g) if act == "silu" else torch.nn.functional.gelu(g, approximate="tanh")
-        h = (gf * u).to(x.dtype)
+        h = _glu_matmul(x2, gate_w, up_w, codec, act, s)
+        if h is None:
+            g, u = quantized_matmul_grouped([(x2, gate_w, codec), (x2, up_w, codec)], out_dtype=torch.float32)
+            gf = torch.nn.functional.silu(g) if act == "silu" else torch.nn.functional.gelu(g, approximate="tanh")
+            h = (gf * u).to(x.dtype)
         y = quantized_matmul(h, down_w, None, down_codec, out_dtype=out_dtype)
     else:
         check("kq_fused_mlp", rc)
     return y.reshape(*x.shape[:-1], N)
+
+
+def _glu_matmul(x2, gate_w, up_w, codec, act, s):
+    """act(x . Wg^T) * (x . Wu^T) in x's dtype in one launch, or None where
+    kq_glu_matmul declines (at most 64 rows)."""
+    L = lib()
+    M, K = x2.shape
+    if M <= 64:
+        return None
+    I, xd = gate_w.shape[0], _dt(x2.dtype)
+    need = L.kq_glu_matmul_workspace_bytes(M, K, xd)
+    ws = _WS.get("matmul", x2.device, s.value, need) if need else None
+    h = torch.empty((M, I), dtype=x2.dtype, device=x2.device)
+    rc = L.kq_glu_matmul(x2.data_ptr(), xd, x2.stride(0), M, K, gate_w.data_ptr(), up_w.data_ptr(), gate_w.stride(0),
+                         _codec_id(codec), I, _lib.ACT_ID[act], h.data_ptr(), xd, h.stride(0),
+                         None if ws is None else ws.data_ptr(), 0 if ws is None else ws.numel(), s)
+    if rc == _lib.KQ_ERR_BAD_SHAPE:
+        return None
+    check("kq_glu_matmul", rc)
+    return h
 
 
 def counts():

@@ -123,8 +123,9 @@ typedef struct {
  *    projections: slices of 8 super-blocks up to 8 rows, 12 past 8) and
  *    Q4_K + Q6_K groups of at most 16 rows (q|k|v: two slices); 17..64-row
  *    groups that the mid-batch streaming kernel takes in slices (the down
- *    projection, q|k|v: 2 or 4 KB per 16-row tile and slice).  The last
- *    slice of each 16-row tile to finish sums the slices in slice order
+ *    projection, q|k|v: 2 or 4 KB per 16-row tile and slice); groups of more
+ *    than 64 rows whose tiles would leave CUs idle (4 bytes per output of a
+ *    tile and slice).  The last slice of each tile to finish sums the slices in slice order
  *    (results stay independent of scheduling).  With fp16 activations a
  *    workspace smaller than this (none included) takes the unsplit kernels
  *    instead. */
@@ -175,6 +176,18 @@ int kq_fused_mlp(const void *x, int x_dtype, int64_t x_row_stride, int32_t M, in
                  const void *w_up, int64_t gu_row_bytes, int gu_codec, int32_t I, const void *w_down,
                  int64_t down_row_bytes, int down_codec, int32_t N, int act, void *y, int y_dtype,
                  int64_t y_row_stride, void *workspace, size_t workspace_bytes, kq_stream_t stream);
+
+/* The gate|up half of the same forward for prompt chunks: h = act(x . Wg^T) *
+ * (x . Wu^T) in fp32, stored as h_dtype, in one launch (bf16 / f32 rows are
+ * prepared first, as for kq_quantized_matmul_grouped; fp16 ones need no
+ * workspace).  gate / up [I, K] wire rows of `codec`, w_row_bytes apart; act:
+ * KQ_ACT_SILU or KQ_ACT_GELU.  Served: more than 64 rows whose fp16 form lies
+ * within 2 GiB; otherwise KQ_ERR_BAD_SHAPE before any launch, and callers run
+ * the grouped matmul and the GLU apart. */
+size_t kq_glu_matmul_workspace_bytes(int32_t M, int32_t K, int x_dtype);
+int kq_glu_matmul(const void *x, int x_dtype, int64_t x_row_stride, int32_t M, int32_t K, const void *w_gate,
+                  const void *w_up, int64_t w_row_bytes, int codec, int32_t I, int act, void *h, int h_dtype,
+                  int64_t h_row_stride, void *workspace, size_t workspace_bytes, kq_stream_t stream);
 
 /* ---- MoE expert gather ------------------------------------------------- */
 /* Device-side routing of (token, slot) pairs to experts.  idx [n_pairs]

@@ -1,0 +1,172 @@
+"""The matrix-core tiles (kq_gemm.hip): dense groups and the dense GLU past 64
+rows, in every tile height and in K slices, and the MoE gathers of long
+segments, against fp64 over the same wire bytes (max |err| / max |ref| within
+the suite's tolerances; fp32 outputs to 1e-5 for Q4_K and IQ2_XXS, whose
+integer codes fp16 holds exactly: what is left is fp32 accumulation over K)."""
+import numpy as np
+import pytest
+
+from helpers import BF16_TOL, TOL, fp16_rows, quantized_weights
+from oracle import kquant as okq
+
+pytestmark = pytest.mark.gpu
+
+CODECS = ("q4_k", "q6_k", "iq2_xxs")
+
+
+def _dev(a):
+    import torch
+    return torch.from_numpy(np.ascontiguousarray(a)).cuda()
+
+
+def _wire(rng, codec, n, k):
+    if codec == "iq2_xxs":
+        return okq.random_valid_blocks(rng, codec, n * k // 256).reshape(n, -1)
+    return quantized_weights(rng, codec, n, k)
+
+
+def _tol(codec):
+    return TOL if codec == "q6_k" else 1e-5
+
+
+@pytest.fixture(autouse=True)
+def _plain(monkeypatch):
+    for k in ("GMLX_KQ_GEMM", "GMLX_KQ_GEMM_MT", "GMLX_KQ_GEMM_S"):
+        monkeypatch.delenv(k, raising=False)
+
+
+# rows and columns on both sides of every tile edge, one super-block up to an
+# odd count; each tile height
+@pytest.mark.parametrize("mt", ["1", "2", "4"])
+@pytest.mark.parametrize("codec", CODECS)
+@pytest.mark.parametrize("M,N,K", [(65, 1, 256), (128, 128, 512), (129, 257, 768), (200, 515, 2816)])
+def test_tiles_match_fp64(codec, M, N, K, mt, monkeypatch):
+    import torch
+    from gmlx_amd import ops
+    monkeypatch.setenv("GMLX_KQ_GEMM_MT", mt)
+    rng = np.random.default_rng(M + N + K)
+    wire, x = _wire(rng, codec, N, K), fp16_rows(rng, M, K)
+    got = ops.quantized_matmul(_dev(x), _dev(wire), None, codec, out_dtype=torch.float32).cpu().numpy()
+    ref = okq.qmm_ref(x, wire, codec)
+    assert okq.max_rel(got, ref) <= _tol(codec), okq.max_rel(got, ref)
+
+
+@pytest.mark.parametrize("dtype_name", ["float16", "bfloat16", "float32"])
+@pytest.mark.parametrize("mt,s", [("2", "3"), ("1", "2"), ("4", "5")])
+def test_k_slices(mt, s, dtype_name, monkeypatch):
+    """A group of two codecs and widths in uneven K slices: fp64, repeats
+    bitwise, counters left zero; rows strided and one-signed."""
+    import torch
+    from gmlx_amd import _lib, ops
+    monkeypatch.setenv("GMLX_KQ_GEMM_MT", mt)
+    monkeypatch.setenv("GMLX_KQ_GEMM_S", s)
+    rng = np.random.default_rng(int(s))
+    M, K = 97, 256 * 23
+    x = (fp16_rows(rng, M, K) + np.float16(2.0)).astype(np.float16)
+    xd = torch.zeros(M, K + 8).to(getattr(torch, dtype_name)).cuda()
+    xd[:, :K] = _dev(x).to(xd.dtype)
+    xd = xd[:, :K]
+    mats = [(_wire(rng, c, n, K), c) for c, n in (("q4_k", 300), ("q6_k", 33))]
+    items = [(xd, _dev(w), c) for w, c in mats]
+    outs = [ops.quantized_matmul_grouped(items, out_dtype=torch.float32) for _ in range(3)]
+    torch.cuda.synchronize()
+    for (w, c), y in zip(mats, outs[0]):
+        ref = okq.qmm_ref(xd.float().cpu().numpy(), w, c)
+        assert okq.max_rel(y.cpu().numpy(), ref) <= TOL, c
+    for o in outs[1:]:
+        assert all(torch.equal(a, b) for a, b in zip(o, outs[0]))
+    ws = ops._WS._ws[("matmul", xd.device.index, ops._stream(xd).value)]
+    assert not ws[:_lib.MATMUL_COUNTER_BYTES].any()
+
+
+def test_slices_replay_in_a_graph():
+    """The plan's own K slices (a down projection of a ragged prompt) captured
+    and replayed between eager calls of another shape, each replay bitwise the
+    eager result."""
+    import torch
+    from gmlx_amd import _lib, ops
+    rng = np.random.default_rng(3)
+    M, N, K = 100, 1024, 12288
+    w, x = _dev(_wire(rng, "q6_k", N, K)), _dev(fp16_rows(rng, M, K))
+    P = _lib.MatmulProblem
+    arr = (P * 1)(P(w.data_ptr(), w.stride(0), x.data_ptr(), K, 1 << 22, N, M, N, K, _lib.CODEC_ID["q6_k"]))
+    assert _lib.lib().kq_matmul_workspace_bytes(arr, 1, _lib.DTYPE_F16) > 0  # slices
+    want = ops.quantized_matmul(x, w, None, "q6_k")
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(s):
+        ops.quantized_matmul(x, w, None, "q6_k")
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=s):
+        y = ops.quantized_matmul(x, w, None, "q6_k")
+    for m in (70, 300, 65):
+        y.zero_()
+        g.replay()
+        other = ops.quantized_matmul(x[:m].contiguous() if m <= M else x.repeat(3, 1), w, None, "q6_k")
+        torch.cuda.synchronize()
+        assert torch.equal(y, want)
+        assert okq.max_rel(other[:65].float().cpu().numpy(), want[:65].float().cpu().numpy()) <= TOL
+
+
+@pytest.mark.parametrize("dtype_name", ["float16", "bfloat16", "float32"])
+@pytest.mark.parametrize("M,I,codec,act,mt", [(65, 128, "q4_k", "silu", "1"), (130, 200, "q6_k", "gelu", "2"),
+                                              (300, 517, "iq2_xxs", "silu", "4")])
+def test_dense_glu(M, I, codec, act, mt, dtype_name, monkeypatch):
+    import torch
+    from gmlx_amd import ops
+    monkeypatch.setenv("GMLX_KQ_GEMM_MT", mt)
+    rng = np.random.default_rng(M)
+    K = 1024
+    gw, uw = _wire(rng, codec, I, K), _wire(rng, codec, I, K)
+    x = _dev(fp16_rows(rng, M, K)).to(getattr(torch, dtype_name))
+    h = ops._glu_matmul(x, _dev(gw), _dev(uw), codec, act, ops._stream(x))
+    xf = x.float().cpu().numpy()
+    g, u = okq.qmm_ref(xf, gw, codec), okq.qmm_ref(xf, uw, codec)
+    a = 0.5 * g * (1 + np.tanh(0.5 * g)) if act == "silu" else \
+        0.5 * g * (1 + np.tanh(0.7978845608028654 * (g + 0.044715 * g ** 3)))
+    assert h.dtype == x.dtype
+    assert okq.max_rel(h.float().cpu().numpy(), a * u) <= (BF16_TOL if dtype_name == "bfloat16" else TOL)
+    assert ops._glu_matmul(x[:64], _dev(gw), _dev(uw), codec, act, ops._stream(x)) is None
+
+
+@pytest.mark.parametrize("mt", ["1", "2"])
+@pytest.mark.parametrize("codec", CODECS)
+def test_long_segments(codec, mt, monkeypatch):
+    """Gathers whose segments are longer than a tile, one row, empty and out of
+    range: plain with a bias, clamped GLU with biases, and the shared-expert
+    layout's spare rows, against the per-tile gathers (GMLX_KQ_GEMM=0) and
+    fp64."""
+    import torch
+    from gmlx_amd import ops
+    rng = np.random.default_rng(11)
+    E, T, k, D, I = 5, 150, 2, 512, 200
+    idx = np.full((T, k), 1)
+    idx[:, 1] = rng.integers(2, 4, T)
+    idx[7] = [0, 5]      # one row for expert 0, an id out of range; expert 4 empty
+    idx[149, 1] = -1
+    w = np.stack([_wire(rng, codec, I, D) for _ in range(E)])
+    wu = np.stack([_wire(rng, codec, I, D) for _ in range(E)])
+    x = fp16_rows(rng, T, D)
+    b0, b1 = (rng.normal(0, 1, (E, I)).astype(np.float32) for _ in range(2))
+    xd, idxd, wd, wud, b0d, b1d = (_dev(a) for a in (x, idx.astype(np.int32), w, wu, b0, b1))
+    sg, su = wd[0].contiguous(), wud[0].contiguous()
+
+    def run(mode):
+        monkeypatch.setenv("GMLX_KQ_GEMM", mode)
+        monkeypatch.setenv("GMLX_KQ_GEMM_MT", mt)
+        y = ops.gather_qmm(xd, wd, None, codec, indices=idxd, out_dtype=torch.float32, bias=b0d)
+        h = ops.moe_glu_gather_kq(xd, wd, wud, codec, idxd, act="swiglu_clamp", gate_bias=b0d, up_bias=b1d)
+        hs = ops.moe_glu_gather_shexp_kq(xd, wd, wud, sg, su, codec, idxd)
+        return y.cpu().numpy(), h.cpu().numpy(), hs.cpu().numpy()
+
+    old, new = run("0"), run("2")
+    for a, b in zip(new, old):
+        assert okq.max_rel(a, b) <= 2e-6 * 16  # fp32 sums in another order
+    ref = np.zeros((T, k, I))
+    for t in range(T):
+        for s in range(k):
+            e = idx[t, s]
+            if 0 <= e < E:
+                ref[t, s] = okq.qmm_ref(x[t:t + 1], w[e], codec)[0] + b0[e]
+    assert okq.max_rel(new[0][:, :, 0], ref) <= _tol(codec)
