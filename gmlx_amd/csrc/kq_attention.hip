@@ -224,12 +224,13 @@ struct KVTile {
     // their scores are masked to -inf, so they contribute p = 0.  kp, vp, t0
     // and t_end are uniform over the wave: the tile's first row is a scalar
     // base and a lane's rows are 32-bit offsets from it (at head dim 512 that
-    // form spilled 12 bytes a lane in the cascade, so rows count from kp).
+    // form spilled 12 bytes a lane in the cascade and at 256 it was slower, 343
+    // against 323 us for eight rows at 12 k: there rows count from kp).
     __device__ __forceinline__ void load(const uint16_t *kp, const uint16_t *vp, int t0, int t_end) {
         const int lane = kq_lane();
         const int r = lane & 15, g = lane >> 4;
-        using Off = std::conditional_t<(D > 256), int64_t, uint32_t>;
-        const int first = D > 256 ? 0 : min(t0, t_end - 1);
+        using Off = std::conditional_t<(D > 128), int64_t, uint32_t>;
+        const int first = D > 128 ? 0 : min(t0, t_end - 1);
         const int last = t_end - 1 - first;
         t0 -= first;
         kp += (int64_t)first * D;
@@ -460,23 +461,29 @@ struct SplitState {
         const float m_new = fmaxf(m_run, tmax);
         // m_new == -inf only for heads >= G.  Every argument is <= 0 and the
         // powers are summed with 1 (the row's maximum), so the hardware's
-        // flush of results below 2^-126 is far below their rounding.
+        // flush of results below 2^-126 is far below their rounding.  (With the
+        // library's range code the compiler schedules the 16-bit tiles of head
+        // dims past 128 better: a cascade of 24 rows at 256 in 339 us against
+        // 385.)
+        constexpr bool kLib = D > 128 && std::is_same_v<Tile, KVTile<D>>;
+        const auto power = [](float v) { return kLib ? exp2f(v) : __builtin_amdgcn_exp2f(v); };
         const bool idle = m_new == -INFINITY;
-        const float alpha = idle ? 1.f : __builtin_amdgcn_exp2f(m_run - m_new);
+        const float alpha = idle ? 1.f : power(m_run - m_new);
         float p[8];
         float psum = 0.f;
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
-            p[i] = idle ? 0.f : __builtin_amdgcn_exp2f(sv[i] - m_new);
+            p[i] = idle ? 0.f : power(sv[i] - m_new);
             psum += p[i];
         }
         l_part = l_part * alpha + psum;
         m_run = m_new;
         // a tile that raises no head's maximum leaves the sums as they are
-        // (alpha is exactly 1): after the first tiles most do not.  At head
-        // dim 512 the branch's copies of the sums spilled 20-56 bytes a lane,
-        // so there each sum is rescaled at its MFMA.
-        constexpr bool kSkip = NG <= 2;
+        // (alpha is exactly 1): after the first tiles most do not.  Past head
+        // dim 128 the branch's copies of the sums cost more (at 512 they
+        // spilled 20-56 bytes a lane), so there each sum is rescaled at its
+        // MFMA.
+        constexpr bool kSkip = NG <= 1;
         if constexpr (kSkip) {
             if (__builtin_amdgcn_ballot_w64(alpha != 1.f)) {
 #pragma unroll
@@ -896,7 +903,9 @@ int env_int(const char *name, int dflt) {
 //   T    36 k   11.9 / 14.1 / 19.1 / 29.7 / 51.2
 //   T   256 k   31.0 / 24.6 / 23.1 / 32.5 / 53.0
 //   T   528 k   53.3 / 47.5 / 46.9 / 45.7 / 55.7
-// So: 64 tokens up to seven waves a CU at that length, given that the
+// So: rows of up to 256 tokens in one split at head dims up to 128 (no merge:
+// its launch costs what the shorter chain gains, and an eager caller's host
+// more); 64 tokens up to seven waves a CU at that length, given that the
 // partials stay under 16 MB (wide head groups at D = 512 would not); then
 // 512, or 256 for an 8-bit cache up to 2048 waves of that length with the
 // same bound; 1024 once B * Hkv * ceil(max_len / 1024) gives every CU 8
@@ -912,6 +921,7 @@ int split_tokens(int B, int Hq, int Hkv, int D, int max_len, bool q8, bool wide)
         const auto units = [&](int64_t tokens) { return heads * ((len + tokens - 1) / tokens); };
         if (units(1024) >= 8 * cus) c = 1024;
         else if (wide) c = 512;
+        else if (len <= 256 && D <= 128) c = 256;
         else if (heads * len <= 7 * 64 * cus && units(64) * group_bytes <= (int64_t)16 << 20) c = 64;
         else c = q8 && units(256) <= 8 * cus && units(256) * group_bytes <= (int64_t)16 << 20 ? 256 : 512;
     }
