@@ -308,7 +308,7 @@ struct RowSums {
     }
     __device__ __forceinline__ void store() const {
         const int g = lane >> 4;
-        const uint32_t key = (uint32_t)(lane & 15) >> 1 & 3u;
+        const uint32_t key = (uint32_t)(lane & 15) >> 2;
         float hi[4], mid[4], lo[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
@@ -612,8 +612,8 @@ __device__ __forceinline__ void setup(Tile<MT, W, GATHER> &t, uint8_t *smem, con
     t.tab = (const Iq2Tables *)(smem + 2 * gemm_x_bytes(MT) + 2 * gemm_sum_bytes(MT));
     t.xs = buffer_words(x, x_bytes);
     t.rd = t.lds + (uint32_t)r * 512u + ((uint32_t)((2 * h) ^ (r & 15)) << 4);
-    // a row's four parts of sums swap places by row, so that eight rows spread over the banks
-    t.sum_rd = t.lds + 2 * gemm_x_bytes(MT) + (uint32_t)r * 64u + ((uint32_t)(h ^ ((r >> 1) & 3)) << 4);
+    // a row's four parts of sums swap places by row, so that sixteen rows spread over the banks
+    t.sum_rd = t.lds + 2 * gemm_x_bytes(MT) + (uint32_t)r * 64u + ((uint32_t)(h ^ ((r >> 2) & 3)) << 4);
 }
 
 template <int MT, int W, bool GATHER>
@@ -963,15 +963,25 @@ int kq_gemm_glu_launch(const kq_matmul_problem &gate, const void *w_up, const in
 bool kq_gemm_gather_eligible(int32_t n_pairs, int32_t n_experts, int64_t x_rows, int64_t x_row_stride) {
     const int mode = env_int("GMLX_KQ_GEMM", 1);
     if (mode == 0 || !addressable(x_rows, x_row_stride)) return false;
-    return mode == 2 || (int64_t)n_pairs >= 8 * (int64_t)n_experts;
+    // The per-tile gathers and the streaming one read a segment's weights in
+    // less time but multiply 8 or 16 rows at a time: measured on whole layers
+    // (us, theirs / these), 128 experts of 2048 x 768: 156 / 169 at 6.2 pairs
+    // per expert, 170 / 173 at 8, 230 / 181 at 12.5, 457 / 258 at 31; 256
+    // IQ2_XXS experts of 7168 x 2048: 1250 / 1632 at 4, 1726 / 1688 at 8,
+    // 3332 / 1912 at 16; 8 experts of 4096 x 6144: 157 / 151 at 4, 197 / 157
+    // at 8.8.
+    return mode == 2 || (int64_t)n_pairs > 8 * (int64_t)n_experts;
 }
 
 int kq_gemm_gather_launch(const KqGemmGather &a, hipStream_t s) {
     const bool glu = a.w1 != nullptr;
-    // rows per tile from the mean segment; the grid bounds every chunk of every segment
+    // Rows per tile from the mean segment: 32 below 28 (a layer at 18.8 rows
+    // per expert: 198 us against 232 with 64-row tiles; at 32 rows 246 against
+    // 195 over 8 experts, 258 against 263 over 128).  The grid bounds every
+    // chunk of every segment.
     const int slots = a.n_experts < a.n_pairs ? a.n_experts : a.n_pairs;
     const int forced = env_int("GMLX_KQ_GEMM_MT", 0);
-    const int mt = forced ? (forced == 1 ? 1 : 2) : a.n_pairs > 20 * (int64_t)slots ? 2 : 1;
+    const int mt = forced ? (forced == 1 ? 1 : 2) : a.n_pairs > 28 * (int64_t)slots ? 2 : 1;
     const int64_t chunks = (int64_t)a.n_pairs / (32 * mt) + slots;
     const int64_t n_tiles = (a.N + tile_cols(mt, glu) - 1) / tile_cols(mt, glu);
     if (chunks * n_tiles > (1 << 28)) return KQ_ERR_BAD_SHAPE;
