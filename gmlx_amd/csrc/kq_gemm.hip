@@ -940,7 +940,8 @@ int kq_gemm_launch(const kq_matmul_problem *ps, const int32_t *const *exps, int 
 }
 
 bool kq_gemm_glu_eligible(const kq_matmul_problem &gate) {
-    return gate.M > 64 && addressable(gate.M, gate.x_row_stride) && env_int("GMLX_KQ_GEMM", 1) != 0;
+    return gate.M > 64 && addressable(gate.M, gate.x_row_stride) && env_int("GMLX_KQ_GEMM", 1) != 0 &&
+           make_plan(&gate, 1, true).mt != 0;
 }
 
 int kq_gemm_glu_launch(const kq_matmul_problem &gate, const void *w_up, const int32_t *x_exp, int act, int y_dtype,
