@@ -3,23 +3,22 @@
 //
 //   y[M, N] = x16[M, K] . dequant(W[N, K])^T,  fp32 accumulation
 //
-// Workgroup: four waves, BM = 32 MT activation rows by 128 NT weight rows;
-// wave w owns 32 NT of the weight rows and all BM activation rows.
+// Workgroup: W waves (eight at MT = 4, four below), BM = 32 MT activation rows
+// by 32 W weight rows (half gate, half up in a GLU launch); a wave owns 32 of
+// the weight rows and all BM activation rows.
 //  - Weights never pass through LDS: a lane holds its weight row's share of a
 //    super-block in registers (half of every 32-value run, 16 contiguous
 //    values) and dequantizes straight into the MFMA operand, so every weight
 //    is decoded once per workgroup.
 //  - Activations do: one super-block (BM rows x 512 bytes) per stage in two
-//    LDS buffers, copied by direct-to-LDS loads one stage ahead; all four
-//    waves read the same rows.  Per v_mfma_f32_32x32x16_f16 a wave reads
-//    1 / NT KB of LDS: at NT = 2, half of what LDS delivers while the four
-//    SIMDs multiply.
+//    LDS buffers, copied by direct-to-LDS loads one stage ahead; every
+//    wave reads the same rows, 1 KB per v_mfma_f32_32x32x16_f16.
 //  - The B operand is the exact integer code of kq_mma.h; each super-block
 //    runs as its own MFMA chain P and folds into the accumulators with the
 //    block's fp32 factor.  Q4_K's minimum term multiplies fp32 sub-block sums
 //    of the activations, held as three bf16 parts (24 bits), by the integer
 //    minimums (exact in bf16) on the matrix cores, and folds with -dmin.
-//    Each wave sums a quarter of the stage's rows; the sums are used one
+//    The waves share the stage's rows out by sixteen; the sums are used one
 //    stage later, behind the stage's only barrier.
 //
 // Lane l = 32 h + r.  Operand layouts of v_mfma_f32_32x32x16: A row / B column
