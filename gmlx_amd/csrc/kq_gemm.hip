@@ -21,6 +21,12 @@
 //    The waves share the stage's rows out by sixteen; the sums are used one
 //    stage later, behind the stage's only barrier.
 //
+// Bound by the matrix cores and the decode that shares the SIMDs with them.
+// Measured against the small-batch dense kernel and the per-tile gathers: an
+// MLP of 2048 bf16 rows (4096 x 12288, Q4_K / Q6_K) 3911 -> 849 us, 725
+// TFLOP/s; the projections of a layer of 333 fp16 rows 832 -> 295 us; an MoE
+// layer of 500 bf16 tokens (128 experts of 2048 x 768, 8 a token) 479 -> 291.
+//
 // Lane l = 32 h + r.  Operand layouts of v_mfma_f32_32x32x16: A row / B column
 // r, k values 8 h .. 8 h + 7; result element i: row 8 (i / 4) + 4 h + i % 4,
 // column r.  Step (sub, half) of a super-block: lane half h covers values
