@@ -50,14 +50,15 @@ typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 __device__ __forceinline__ u32x4 lds128(uint32_t a) { return *(const LDSP(u32x4))(uintptr_t)a; }
 
 // 16 bytes a lane from buffer `rs` at voff + soff straight to LDS (lane l's at
-// lds + 16 l).  Written out because the compiler, seeing the builtin, orders
+// lds + 16 l; the base goes in m0, an operand so that the compiler knows what
+// m0 holds).  Written out because the compiler, seeing the builtin, orders
 // every LDS read behind it and would drain the copy of the next stage before
 // the first fragment of this one; the wait is the explicit one at the stage's
 // barrier.  No register receives the load.
 __device__ __forceinline__ void dma16(u32x4 rs, uint32_t lds, uint32_t voff, uint32_t soff) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+    asm volatile("s_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
                  :
-                 : "s"(lds), "v"(voff), "s"(rs), "s"(soff));
+                 : "{m0}"(lds), "v"(voff), "s"(rs), "s"(soff));
 }
 
 // Raw buffer descriptor over `bytes` bytes at `base`, in scalar registers.

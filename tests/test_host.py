@@ -324,3 +324,22 @@ def test_install_kquant_modules_swaps_embeddings_and_expert_stacks(monkeypatch):
     assert knn.install_kquant_modules(model, {"emb.weight": "q6_k"}) == 0   # already swapped
     monkeypatch.setenv("GMLX_ACTIVATION_DTYPE", "auto")
     assert knn.activation_dtype() == torch.bfloat16
+
+
+def test_inline_assembly_declares_its_use_of_m0():
+    """Inline assembly whose instructions write m0, or copy to LDS (the base is
+    in m0), says so in its operands or clobbers: the compiler keeps the LDS
+    base of its own copies in m0 across an asm block that does not."""
+    csrc = os.path.join(ROOT, "gmlx_amd", "csrc")
+    found = 0
+    for name in sorted(os.listdir(csrc)):
+        text = open(os.path.join(csrc, name)).read()
+        for stmt in re.findall(r"\basm(?:\s+volatile)?\s*\((.*?)\)\s*;", text, flags=re.S):
+            code = re.match(r'\s*"(?:[^"\\]|\\.)*"', stmt).group(0)
+            operands = stmt[len(code):]
+            if not re.search(r"\bm0\b|\blds\b", code):
+                continue
+            found += 1
+            writes = re.search(r"\bs_\w+\s+m0\b", code)
+            assert ('"m0"' in operands) if writes else ('"{m0}"' in operands), (name, stmt)
+    assert found  # kq_gemm.hip's copies
