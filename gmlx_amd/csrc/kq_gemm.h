@@ -19,7 +19,8 @@ bool kq_gemm_glu_eligible(const kq_matmul_problem &gate);
 int kq_gemm_glu_launch(const kq_matmul_problem &gate, const void *w_up, const int32_t *x_exp, int act, int y_dtype,
                        hipStream_t s);
 
-// The MoE gathers (kq_moe_gather_rows): w1 null for the plain form.
+// The MoE gathers (kq_moe_gather_rows): w1 null for the plain form.  x: x_rows
+// fp16 rows; streams: the streaming gather would take the call otherwise.
 struct KqGemmGather {
     const char *x;
     const int32_t *x_exp;
@@ -32,5 +33,5 @@ struct KqGemmGather {
     int32_t x_pair_div, x_skip, y_skip, N, K, codec, n_pairs, n_experts, y_dtype, act;
     float limit, alpha;
 };
-bool kq_gemm_gather_eligible(int32_t n_pairs, int32_t n_experts, int64_t x_rows, int64_t x_row_stride);
+bool kq_gemm_gather_eligible(const KqGemmGather &a, int64_t x_rows, int64_t x_row_stride, bool streams);
 int kq_gemm_gather_launch(const KqGemmGather &a, hipStream_t s);

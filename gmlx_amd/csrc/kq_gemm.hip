@@ -967,28 +967,72 @@ int kq_gemm_glu_launch(const kq_matmul_problem &gate, const void *w_up, const in
     return launch_mt<true>(plan.mt, a, s);
 }
 
-bool kq_gemm_gather_eligible(int32_t n_pairs, int32_t n_experts, int64_t x_rows, int64_t x_row_stride) {
+// Rows per tile of a gather from the mean segment: 32 up to 28 (a layer at
+// 18.8 rows per expert: 198 us against 232 with 64-row tiles), 64 past it (at
+// 32 rows over 8 experts 195 us against 246; over 128 experts the two are
+// level, 263 against 258).
+static int gather_mt(int64_t n_pairs, int slots) {
+    const int forced = env_int("GMLX_KQ_GEMM_MT", 0);
+    return forced ? (forced == 1 ? 1 : 2) : n_pairs > 28 * (int64_t)slots ? 2 : 1;
+}
+
+// Whether a gather is shorter on these tiles than on the kernel it would take
+// otherwise (`streams`: the streaming gather, else the per-tile ones).
+//
+// Those read a segment's weights in less time but multiply 8 or 16 rows at a
+// time.  Launches of more tiles than CUs, whole layers (us, theirs / these):
+// 128 experts of 2048 x 768, 156 / 169 at 6.2 pairs per expert, 170 / 173 at
+// 8, 230 / 181 at 12.5, 457 / 258 at 31; 256 IQ2_XXS experts of 7168 x 2048,
+// 1250 / 1632 at 4, 1726 / 1688 at 8, 3332 / 1912 at 16; 16 IQ2_XXS experts
+// of 4096 x 1024, 45 / 51 at 8.5, 55 / 52 at 12.  So the line is 8 pairs per
+// expert, 10 for IQ2_XXS.
+//
+// A launch of at most one tile a CU (few experts or narrow ones, above all the
+// shared expert, one segment of all the tokens) is one tile's walk over K
+// long, while the other kernels cut N by sixteens and long K over four waves:
+// there both times are estimated, and the tiles have to win by 8 %.  Fitted to
+// 374 launches (1 to 16 experts, 8.5 to 1024 rows each, N 512 to 8192, K 512
+// to 8192, the three codecs) and tried on 160 more: 188 of the 374 ran over
+// 3 % slower on these tiles, by up to 4.2 times; with the rule 4 of all 534 do,
+// by 4 to 15 %.  Theirs / these, one expert's
+// GLU of 768 x 2048 in Q4_K: 9.1 / 19.0 at 24 rows, 22 / 29 at 256, 36 / 30 at
+// 512; 2048 x 7168: 23 / 41, 152 / 62 and 299 / 71; its down projection in
+// Q6_K: 24 / 26, 146 / 36 and 287 / 51.
+static bool gather_pays(const KqGemmGather &a, bool streams) {
+    const bool q6 = a.codec == KQ_CODEC_Q6_K, iq2 = a.codec == KQ_CODEC_IQ2_XXS, glu = a.w1 != nullptr;
+    if (a.n_pairs <= (iq2 ? 10 : 8) * (int64_t)a.n_experts) return false;
+    const int cus = device_cus(), slots = a.n_experts < a.n_pairs ? a.n_experts : a.n_pairs;
+    const double mean = (double)a.n_pairs / slots;
+    const int mt = gather_mt(a.n_pairs, slots);
+    const int64_t n_tiles = (a.N + tile_cols(mt, glu) - 1) / tile_cols(mt, glu);
+    if (slots * (1 + (int64_t)((a.n_pairs - 1) / ((int64_t)slots * 32 * mt))) * n_tiles > cus) return true;
+    const double nb = a.K / KQ_QK;
+    const double tiles = mt == 1 ? 10 + nb * (q6 ? 2.05 : iq2 ? 1.4 : 1.1) : 13 + nb * (q6 ? 2.5 : iq2 ? 1.75 : 1.6);
+    double theirs;
+    if (streams) {
+        // by the weights read and the rows multiplied, per 2 x 768 x 2048 weights of an expert
+        theirs = 8 + 2.0 * a.N * a.K / (2.0 * 768 * 2048) * (0.35 * slots + 0.07 * a.n_pairs);
+    } else {
+        // a unit's chunks of 16 rows (segments scatter about the mean) by its
+        // steps through K, times the rounds of units
+        const int chunks = slots == 1 ? (a.n_pairs + 15) / 16 : (int)(mean / 16) + 1;
+        const double waves = (double)slots * ((a.N + 15) / 16) * (nb > 8 ? 4 : 1) * (glu ? 1.5 : 1.0) *
+                             (iq2 ? 0.8 : 1.0) / (4.0 * cus);
+        theirs = 7 + 1.2 * chunks * (nb > 8 ? nb / 4 : nb) * (waves > 1 ? waves : 1);
+    }
+    return theirs > 1.08 * tiles;
+}
+
+bool kq_gemm_gather_eligible(const KqGemmGather &a, int64_t x_rows, int64_t x_row_stride, bool streams) {
     const int mode = env_int("GMLX_KQ_GEMM", 1);
-    if (mode == 0 || !addressable(x_rows, x_row_stride)) return false;
-    // The per-tile gathers and the streaming one read a segment's weights in
-    // less time but multiply 8 or 16 rows at a time: measured on whole layers
-    // (us, theirs / these), 128 experts of 2048 x 768: 156 / 169 at 6.2 pairs
-    // per expert, 170 / 173 at 8, 230 / 181 at 12.5, 457 / 258 at 31; 256
-    // IQ2_XXS experts of 7168 x 2048: 1250 / 1632 at 4, 1726 / 1688 at 8,
-    // 3332 / 1912 at 16; 8 experts of 4096 x 6144: 157 / 151 at 4, 197 / 157
-    // at 8.8.
-    return mode == 2 || (int64_t)n_pairs > 8 * (int64_t)n_experts;
+    return mode != 0 && addressable(x_rows, x_row_stride) && (mode == 2 || gather_pays(a, streams));
 }
 
 int kq_gemm_gather_launch(const KqGemmGather &a, hipStream_t s) {
     const bool glu = a.w1 != nullptr;
-    // Rows per tile from the mean segment: 32 below 28 (a layer at 18.8 rows
-    // per expert: 198 us against 232 with 64-row tiles; at 32 rows 246 against
-    // 195 over 8 experts, 258 against 263 over 128).  The grid bounds every
-    // chunk of every segment.
+    // the grid bounds every chunk of every segment
     const int slots = a.n_experts < a.n_pairs ? a.n_experts : a.n_pairs;
-    const int forced = env_int("GMLX_KQ_GEMM_MT", 0);
-    const int mt = forced ? (forced == 1 ? 1 : 2) : a.n_pairs > 28 * (int64_t)slots ? 2 : 1;
+    const int mt = gather_mt(a.n_pairs, slots);
     const int64_t chunks = (int64_t)a.n_pairs / (32 * mt) + slots;
     const int64_t n_tiles = (a.N + tile_cols(mt, glu) - 1) / tile_cols(mt, glu);
     if (chunks * n_tiles > (1 << 28)) return KQ_ERR_BAD_SHAPE;

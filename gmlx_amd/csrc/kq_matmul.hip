@@ -1035,42 +1035,41 @@ int gather_common(const void *x, int x_dtype, int64_t x_row_stride, int32_t x_pa
         x_row_stride = K;
         x_dtype = KQ_DTYPE_F16;
     }
-    // long segments: the matrix-core tiles
-    const int32_t x_rows = gather_x_rows(n_pairs, x_pair_div, x_skip);
-    if (kq_gemm_gather_eligible(n_pairs, n_experts, x_rows, x_row_stride)) {
-        KqGemmGather g;
-        g.x = (const char *)x;
-        g.x_exp = x_exp;
-        g.w0 = (const uint8_t *)w0;
-        g.w1 = (const uint8_t *)w1;
-        g.y = y;
-        g.seg_info = seg_info;
-        g.pair_order = pair_order;
-        g.b0 = ep->bias0;
-        g.b1 = w1 ? ep->bias1 : nullptr;
-        g.w_expert_bytes = w_expert_bytes;
-        g.w_row_bytes = w_row_bytes;
-        g.y_stride = y_row_stride;
-        g.b_stride = ep->bias_expert_stride;
-        g.x_row_bytes = (uint32_t)x_row_stride * 2;
-        g.x_bytes = (uint32_t)(((int64_t)(x_rows - 1) * x_row_stride + K) * 2);
-        g.x_pair_div = x_pair_div;
-        g.x_skip = x_skip;
-        g.y_skip = y_skip;
-        g.N = N;
-        g.K = K;
-        g.codec = codec;
-        g.n_pairs = n_pairs;
-        g.n_experts = n_experts;
-        g.y_dtype = y_dtype;
-        g.act = w1 ? ep->act : KQ_ACT_SILU;
-        g.limit = ep->limit;
-        g.alpha = ep->alpha;
-        return kq_gemm_gather_launch(g, s);
-    }
     // the streaming gather: weight tiles by row-contiguous direct-to-LDS
     // copies, one persistent workgroup per CU
-    if (kq_sgather_eligible(codec, w1 != nullptr, N, K, w_row_bytes, n_experts))
+    const bool streams = kq_sgather_eligible(codec, w1 != nullptr, N, K, w_row_bytes, n_experts);
+    // long segments: the matrix-core tiles
+    const int32_t x_rows = gather_x_rows(n_pairs, x_pair_div, x_skip);
+    KqGemmGather g;
+    g.x = (const char *)x;
+    g.x_exp = x_exp;
+    g.w0 = (const uint8_t *)w0;
+    g.w1 = (const uint8_t *)w1;
+    g.y = y;
+    g.seg_info = seg_info;
+    g.pair_order = pair_order;
+    g.b0 = ep->bias0;
+    g.b1 = w1 ? ep->bias1 : nullptr;
+    g.w_expert_bytes = w_expert_bytes;
+    g.w_row_bytes = w_row_bytes;
+    g.y_stride = y_row_stride;
+    g.b_stride = ep->bias_expert_stride;
+    g.x_row_bytes = (uint32_t)x_row_stride * 2;
+    g.x_bytes = (uint32_t)(((int64_t)(x_rows - 1) * x_row_stride + K) * 2);
+    g.x_pair_div = x_pair_div;
+    g.x_skip = x_skip;
+    g.y_skip = y_skip;
+    g.N = N;
+    g.K = K;
+    g.codec = codec;
+    g.n_pairs = n_pairs;
+    g.n_experts = n_experts;
+    g.y_dtype = y_dtype;
+    g.act = w1 ? ep->act : KQ_ACT_SILU;
+    g.limit = ep->limit;
+    g.alpha = ep->alpha;
+    if (kq_gemm_gather_eligible(g, x_rows, x_row_stride, streams)) return kq_gemm_gather_launch(g, s);
+    if (streams)
         return kq_sgather_launch(x, x_exp, x_row_stride, x_pair_div, x_skip, w0, w1, w_expert_bytes, w_row_bytes, N,
                                  K, codec, w1 ? ep->act : KQ_ACT_SILU, ep->limit, ep->alpha, ep->bias0,
                                  w1 ? ep->bias1 : nullptr, ep->bias_expert_stride, seg_info, pair_order, n_pairs,

@@ -170,3 +170,31 @@ def test_long_segments(codec, mt, monkeypatch):
             if 0 <= e < E:
                 ref[t, s] = okq.qmm_ref(x[t:t + 1], w[e], codec)[0] + b0[e]
     assert okq.max_rel(new[0][:, :, 0], ref) <= _tol(codec)
+
+
+@pytest.mark.parametrize("T,tiles", [(9, False), (33, False), (512, True)])
+def test_one_expert_takes_the_tiles_only_when_they_fill_the_gpu(T, tiles, monkeypatch):
+    """A shared expert's GLU and down gathers (one expert of 768 x 2048: 12 to
+    96 tiles on 256 CUs): the default call's bits are those of the small-batch
+    gathers at 9 and 33 tokens, of the tiles at 512, where they are faster."""
+    import torch
+    from gmlx_amd import ops
+    rng = np.random.default_rng(T)
+    D, I = 2048, 768
+    gw, uw, dw = (_dev(okq.random_valid_blocks(rng, "q4_k", n * k // 256).reshape(1, n, -1))
+                  for n, k in ((I, D), (I, D), (D, I)))
+    x = _dev(fp16_rows(rng, T, D))
+    h = _dev(fp16_rows(rng, T, I)).reshape(T, 1, I)
+    idx = torch.zeros(T, 1, dtype=torch.int32, device="cuda")
+
+    def run():
+        return (ops.moe_glu_gather_kq(x, gw, uw, "q4_k", idx), ops.gather_qmv_kq(h, dw, "q4_k", idx))
+
+    got = run()
+    outs = {}
+    for mode in ("0", "2"):
+        monkeypatch.setenv("GMLX_KQ_GEMM", mode)
+        outs[mode] = run()
+    for a, old, new in zip(got, outs["0"], outs["2"]):
+        assert not torch.equal(old, new)
+        assert torch.equal(a, new if tiles else old)
