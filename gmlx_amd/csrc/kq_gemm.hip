@@ -918,10 +918,37 @@ bool addressable(int64_t rows, int64_t row_stride) { return rows * row_stride * 
 
 }  // namespace
 
+// Small launches of short rows stay on the dense kernel: fewer than 8
+// super-blocks take no K slices, so a launch is one tile's walk over K long,
+// and a Q6_K step takes 1.6 us here against 1.3 there, as long as that
+// kernel's workgroups (32 columns by 64 rows) fit one a CU.  Theirs / these,
+// 65 to 128 rows (us): Q6_K, 1024 rows of 256 values 8.7 / 8.9, of 1024 12.6 /
+// 13.8, of 1792 17.1 / 22.1, of 2048 (two slices) 18.1 / 16.2; 4096 rows of
+// 1024 13.0 / 14.5, and 18.6 / 14.6 at 129 rows, where they no longer fit; a
+// q|k|v group (Q4_K, V in Q6_K) of 4096 rows of 1024 13.0 / 14.5; IQ2_XXS, 512
+// rows of 1536 13.6 / 14.8, of 1024 11.7 / 11.8.  Everywhere else past 64 rows
+// the tiles are level or ahead: 65 rows by 4096 x 4096 28.8 / 20.2 in Q4_K,
+// 28.6 / 24.1 in Q6_K, 25.1 / 20.4 in IQ2_XXS; 12288 x 4096 68 / 33, 74 / 49,
+// 58 / 33; Q4_K by 1024 x 1024 12.2 / 10.1.
+static bool dense_kernel_pays(const kq_matmul_problem *ps, int n) {
+    bool slow = false;
+    int64_t workgroups = 0;
+    for (int i = 0; i < n; ++i) {
+        const int nb = ps[i].K / KQ_QK;
+        if (nb >= 8) return false;
+        slow = slow || ps[i].codec == KQ_CODEC_Q6_K || (ps[i].codec == KQ_CODEC_IQ2_XXS && nb > 4);
+        workgroups += (int64_t)((ps[i].N + 31) / 32) * ((ps[i].M + 63) / 64);
+    }
+    return slow && workgroups <= device_cus();
+}
+
 bool kq_gemm_eligible(const kq_matmul_problem *ps, int n) {
     for (int i = 0; i < n; ++i)
         if (ps[i].M <= 64 || !addressable(ps[i].M, ps[i].x_row_stride)) return false;
-    return n > 0 && env_int("GMLX_KQ_GEMM", 1) != 0 && make_plan(ps, n, false).mt != 0;
+    const int mode = env_int("GMLX_KQ_GEMM", 1);
+    if (n <= 0 || mode == 0) return false;
+    if (mode != 2 && !env_int("GMLX_KQ_GEMM_MT", 0) && dense_kernel_pays(ps, n)) return false;
+    return make_plan(ps, n, false).mt != 0;
 }
 
 size_t kq_gemm_part_bytes(const kq_matmul_problem *ps, int n) {

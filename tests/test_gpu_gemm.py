@@ -198,3 +198,26 @@ def test_one_expert_takes_the_tiles_only_when_they_fill_the_gpu(T, tiles, monkey
     for a, old, new in zip(got, outs["0"], outs["2"]):
         assert not torch.equal(old, new)
         assert torch.equal(a, new if tiles else old)
+
+
+@pytest.mark.parametrize("M,mats,tiles", [
+    (100, [("q6_k", 1000)], False), (65, [("q4_k", 2048), ("q4_k", 1024), ("q6_k", 1024)], False),
+    (100, [("iq2_xxs", 300)], False), (300, [("q6_k", 3072)], True), (100, [("q4_k", 1000)], True)])
+def test_short_rows_take_the_tiles_only_past_one_round(M, mats, tiles, monkeypatch):
+    """Groups of rows shorter than 8 super-blocks with Q6_K or IQ2_XXS among
+    them: the default call's bits are the dense kernel's while its workgroups
+    fit one a CU, else the tiles'."""
+    import torch
+    from gmlx_amd import ops
+    rng = np.random.default_rng(M)
+    K = 1536 if mats[0][0] == "iq2_xxs" else 1024
+    x = _dev(fp16_rows(rng, M, K))
+    items = [(x, _dev(okq.random_valid_blocks(rng, c, n * K // 256).reshape(n, -1)), c) for c, n in mats]
+    got = ops.quantized_matmul_grouped(items, out_dtype=torch.float32)
+    outs = {}
+    for mode in ("0", "2"):
+        monkeypatch.setenv("GMLX_KQ_GEMM", mode)
+        outs[mode] = ops.quantized_matmul_grouped(items, out_dtype=torch.float32)
+    for a, dense, tile in zip(got, outs["0"], outs["2"]):
+        assert not torch.equal(dense, tile)
+        assert torch.equal(a, tile if tiles else dense)
