@@ -39,6 +39,15 @@ int device_cus();
 
 namespace {
 
+// Tokens per split of a ragged row, by the row's own length (split_rule).
+struct SplitRule {
+    int32_t one, to64, to128, to256, rest;
+
+    __host__ __device__ __forceinline__ int tokens(int len) const {
+        return len <= one ? one : len <= to64 ? 64 : len <= to128 ? 128 : len <= to256 ? 256 : rest;
+    }
+};
+
 struct SdpaArgs {
     const uint16_t *q, *k, *v;
     uint16_t *out;
@@ -55,7 +64,9 @@ struct SdpaArgs {
     int32_t split1;             // tokens per prefix split
     float *part;          // [B][Hkv][max_splits][G][D] O partials
     float *ml;            // [B][Hkv][max_splits][G][2] (m, l)
-    int32_t B, Hq, Hkv, G, split, max_splits, max_len;
+    int32_t B, Hq, Hkv, G, max_splits, max_len;
+    SplitRule rule;       // ragged mode
+    int32_t split;        // cascade mode: tokens per private split
     int32_t qL;           // query tokens per sequence: row r is token r % qL of sequence r / qL
     // 8-bit affine KV (q8 != 0): k / v (k2 / v2) hold uint8 values, token
     // rows of D bytes, offsets and strides in bytes; ks / kb / vs / vb (and
@@ -72,7 +83,7 @@ struct SdpaArgs {
     int32_t padded;
     int64_t pad_batch_stride, pad_head_stride;
     // direct != 0 (padded mode): the split grid is (split, kv head, row), so a
-    // wave finds its unit without the scan over the rows' split counts
+    // wave finds its units without the scan over the rows' split counts
     int32_t direct;
 };
 
@@ -116,7 +127,7 @@ __device__ __forceinline__ int padded_start(const SdpaArgs &a, int b) {
 }
 
 // Keys of ragged row b (rows longer than max_len are clamped to it: the
-// workspace holds max_len / split splits per (row, head)).
+// workspace holds max_splits splits per (row, head)).
 __device__ __forceinline__ int ragged_len(const SdpaArgs &a, int b) {
     if (a.padded) return a.max_len - padded_start(a, b);
     return max(min(a.row_len[b], a.max_len), 0);
@@ -129,7 +140,8 @@ __device__ __forceinline__ int64_t ragged_base(const SdpaArgs &a, int b, int h, 
     return a.kv_off[b] + (int64_t)h * a.head_stride[b];
 }
 
-__device__ __forceinline__ int row_splits(int len, int split) {
+__host__ __device__ __forceinline__ int row_splits(const SplitRule &rule, int len) {
+    const int split = rule.tokens(len);
     return len <= 0 ? 1 : (len + split - 1) / split;
 }
 
@@ -147,7 +159,7 @@ __device__ __forceinline__ int cascade_len2(const SdpaArgs &a, int r) {
 // splits; cascade mode, the private slab's (the prefix units are counted
 // apart).  A row with no keys keeps one (empty) split.
 __device__ __forceinline__ int row_unit_splits(const SdpaArgs &a, int b) {
-    if (!a.cascade) return row_splits(ragged_len(a, b), a.split);
+    if (!a.cascade) return row_splits(a.rule, ragged_len(a, b));
     const int n2 = (cascade_len2(a, b) + a.split - 1) / a.split;
     return a.n1 == 0 ? max(n2, 1) : n2;
 }
@@ -716,7 +728,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(D <= 128 ? 2
     for (int u = blockIdx.x;; u += gridDim.x) {
         int b, h, s;
         if (a.direct) {
-            // grid (split, kv head, row): one unit per workgroup
+            // grid (split, kv head, row)
             s = u;
             h = blockIdx.y;
             b = blockIdx.z;
@@ -725,14 +737,14 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(D <= 128 ? 2
             return;
         }
         const int len = ragged_len(a, b);
-        const int t_begin = s * a.split;
-        const int t_end = min(len, t_begin + a.split);
+        const int split = a.rule.tokens(len);
+        const int t_begin = s * split;
+        const int t_end = min(len, t_begin + split);
         const int64_t kvbase = ragged_base(a, b, h, D);
         const int rw[1] = {b}, hd[1] = {r < a.G ? r : 0};
         const bool ok[1] = {r < a.G};
         split_unit<D, BF, NBUF, 1, Q8>(a, kv_src<Q8>(a.k, a.v, a.ks, a.kb, a.vs, a.vb, kvbase), t_begin, t_end, h, s,
                                        rw, hd, ok, q_lds);
-        if (a.direct) return;
     }
 }
 
@@ -888,66 +900,75 @@ int env_int(const char *name, int dflt) {
     return (end && *end == 0 && v > 0 && v < (1 << 24)) ? (int)v : dflt;
 }
 
-// Tokens per split (a multiple of the 32-token tile), by the launch's size in
-// head-tokens T = B * Hkv * max_len (max_len bounds every row).  A split is
-// one wave's chain of tiles, 0.5-0.8 us each, and one fp32 partial to write
-// and merge: short launches want short chains, long ones few partials.
-// Measured per call, D = 128 (us at 64 / 128 / 256 / 512 / 1024 tokens),
-// 16-bit:
-//   T    16 k   9.2 / 10.3 / 12.8 / 18.0 / 28.1
-//   T    36 k   11.4 / 11.5 / 13.4 / 18.7 / 28.7
-//   T   118 k   24.7 / 22.6 / 20.6 / 21.5 / 29.8
-//   T   256 k   37.3 / 32.9 / 31.5 / 30.5 / 32.1
-//   T 1 024 k   119.4 / 115.1 / 109.4 / 102.7 / 98.9
-// and over an 8-bit cache with bf16 queries
-//   T    36 k   11.9 / 14.1 / 19.1 / 29.7 / 51.2
-//   T   256 k   31.0 / 24.6 / 23.1 / 32.5 / 53.0
-//   T   528 k   53.3 / 47.5 / 46.9 / 45.7 / 55.7
-// So: rows of up to 256 tokens in one split at head dims up to 128 (no merge:
-// its launch costs what the shorter chain gains, and an eager caller's host
-// more); 64 tokens up to seven waves a CU at that length, given that the
-// partials stay under 16 MB (wide head groups at D = 512 would not); then
-// 512, or 256 for an 8-bit cache up to 2048 waves of that length with the
-// same bound; 1024 once B * Hkv * ceil(max_len / 1024) gives every CU 8
-// waves.  `wide` keeps to 512 and 1024: the plan of a call whose workspace
-// is too small for the short splits' partials.  GMLX_KQ_SDPA_SPLIT forces
-// one length.  The workspace size follows the same rule from the same
-// arguments.
-int split_tokens(int B, int Hq, int Hkv, int D, int max_len, bool q8, bool wide) {
-    int c = env_int("GMLX_KQ_SDPA_SPLIT", 0);
-    if (c == 0) {
-        const int64_t group_bytes = (int64_t)(Hq / Hkv) * D * 4;
-        const int64_t heads = (int64_t)B * Hkv, len = max_len > 0 ? max_len : 1, cus = device_cus();
-        const auto units = [&](int64_t tokens) { return heads * ((len + tokens - 1) / tokens); };
-        if (units(1024) >= 8 * cus) c = 1024;
-        else if (wide) c = 512;
-        else if (len <= 256 && D <= 128) c = 256;
-        else if (heads * len <= 7 * 64 * cus && units(64) * group_bytes <= (int64_t)16 << 20) c = 64;
-        else c = q8 && units(256) <= 8 * cus && units(256) * group_bytes <= (int64_t)16 << 20 ? 256 : 512;
+// Tokens per split (multiples of the 32-token tile).  A split is one wave's
+// chain of tiles, 0.5-0.8 us each, and one fp32 partial to write and merge:
+// short launches want short chains, long ones few partials.  The length
+// follows from the row's own keys and from what all calls on a cache share
+// (head counts, D, 16 or 8 bits), not from the batch around the row: a row's
+// bits are those of the call on the row alone.  So it has to suit one row and
+// many.  Measured per call, 8 kv heads, D = 128 (us at 64 / 128 / 256 / 512
+// tokens; rows of equal length), 16-bit with four query heads a kv head:
+//   1 row of  400   8.0 / 9.5 / 11.9 / 12.2      32 rows  19.2 / 19.5 / 18.4 / 14.4
+//   1 row of 1600   9.0 / 10.1 / 12.7 / 17.6     32 rows  54.4 / 53.6 / 50.0 / 49.7
+//   1 row of 6400   14.5 / 13.5 / 13.7 / 18.4    16 rows  93.7 / 90.9 / 94.5 / 88.2
+//   1 of 12800      21.7 / 19.6 / 18.4 / 19.1     8 rows  94.8 / 91.1 / 95.7 / 89.0
+// with sixteen
+//   1 row of 1600   9.5 / 10.2 / 12.8 / 17.9     32 rows  71.0 / 63.6 / 58.3 / 58.7
+// over an 8-bit cache
+//   1 row of  800   9.9 / 12.7 / 18.2 / 28.9     32 rows  26.4 / 22.9 / 23.4 / 32.9
+//   1 row of 3200   12.6 / 13.6 / 19.0 / 29.7    32 rows  73.4 / 64.8 / 63.1 / 58.9
+//   1 of 32768      37.0 / 28.6 / 24.7 / 33.1     3 rows  74.9 / 64.0 / 58.2 / 56.7
+// and at D = 256, two query heads
+//   1 row of 1600   12.5 / 14.4 / 20.8 / 33.6    32 rows  93.8 / 92.4 / 90.1 / 84.7
+// So: up to 256 tokens one split (no merge; 512 past four query heads a kv
+// head, whose merges cost as many times more; 128 at D = 256, none past it or
+// there in 8 bits); then 64, 128 and 256 up to the lines below, past them 512.
+// Against 512 throughout, 376 launches of 1 to 32 equal rows took 0.66 times
+// as long in the geometric mean; 47 took over 3 % longer, 46 of them by at
+// most 13 % and 32 rows of 400 tokens 19 us against 14.5: there the merge
+// costs more than the shorter chain gives, and with one row it is 8 against 12.
+// A launch of B * Hkv * ceil(max_len / 1024) >= 8 waves a CU takes 1024 for
+// every row (C3: 353 against 372 us at 512): a row's bits there are not those
+// of the row alone.  `wide` keeps to 512 and 1024: the plan
+// of a call whose workspace is too small for the partials of the short splits.
+// GMLX_KQ_SDPA_SPLIT forces one length.  The workspace size follows the same
+// rule from the same arguments.
+SplitRule split_rule(int B, int Hq, int Hkv, int D, int max_len, bool q8, bool wide) {
+    SplitRule r{0, 0, 0, 0, 512};
+    const int forced = env_int("GMLX_KQ_SDPA_SPLIT", 0);
+    if (forced) {
+        r.rest = forced <= 32 ? 32 : (forced + 31) / 32 * 32;
+    } else if ((int64_t)B * Hkv * (((int64_t)(max_len > 0 ? max_len : 1) + 1023) / 1024) >= 8 * (int64_t)device_cus()) {
+        r.rest = 1024;
+    } else if (!wide) {
+        if (D > 128) r = SplitRule{q8 || D > 256 ? 0 : 128, 1024, 8192, 32768, 512};
+        else if (q8) r = SplitRule{256, 1024, 2048, 32768, 512};
+        else r = Hq > 4 * Hkv ? SplitRule{512, 0, 1024, 8192, 512} : SplitRule{256, 512, 4096, 8192, 512};
     }
-    c = (c + 31) / 32 * 32;
-    return c < 32 ? 32 : c;
+    return r;
 }
 
 struct WsLayout {
     size_t part_bytes, ml_bytes;
-    int split;
+    SplitRule rule;
+    int max_splits;  // of any row of at most max_len keys
+
+    size_t bytes() const { return part_bytes + ml_bytes; }
 };
 
 WsLayout ws_layout(int B, int Hq, int Hkv, int D, int max_len, bool q8, bool wide = false) {
-    const int G = Hq / Hkv;
-    const int C = split_tokens(B, Hq, Hkv, D, max_len, q8, wide);
-    const int64_t ms = max_len <= 0 ? 1 : (max_len + C - 1) / C;
     WsLayout w;
-    w.split = C;
-    w.part_bytes = (((size_t)B * Hkv * ms * G * D * 4) + 255) & ~(size_t)255;
-    w.ml_bytes = (size_t)B * Hkv * ms * G * 2 * 4;
+    w.rule = split_rule(B, Hq, Hkv, D, max_len, q8, wide);
+    // the most splits are those of max_len or of a row at a line below it
+    w.max_splits = row_splits(w.rule, max_len);
+    for (const int line : {w.rule.one, w.rule.to64, w.rule.to128, w.rule.to256}) {
+        const int n = line < max_len ? row_splits(w.rule, line) : 1;
+        if (n > w.max_splits) w.max_splits = n;
+    }
+    const size_t slots = (size_t)B * Hkv * w.max_splits * (Hq / Hkv);
+    w.part_bytes = (slots * D * 4 + 255) & ~(size_t)255;
+    w.ml_bytes = slots * 2 * 4;
     return w;
-}
-
-size_t ws_bytes(int B, int Hq, int Hkv, int D, int max_len, bool q8) {
-    const WsLayout w = ws_layout(B, Hq, Hkv, D, max_len, q8);
-    return w.part_bytes + w.ml_bytes;
 }
 
 // Row blocks per prefix wave: 2 (GMLX_KQ_CASCADE_NRB=1 selects one).  Four
@@ -972,7 +993,7 @@ void launch_n(const SdpaArgs &a, int grid, int block, bool merge, hipStream_t s)
         }
     } else
         hipLaunchKernelGGL((kq_sdpa_split_kernel<D, BF, NBUF, Q8>),
-                           a.direct ? dim3(a.max_splits, a.Hkv, a.B) : dim3(grid), dim3(64), 0, s, a);
+                           a.direct ? dim3(grid, a.Hkv, a.B) : dim3(grid), dim3(64), 0, s, a);
     if (merge) hipLaunchKernelGGL((kq_sdpa_merge_kernel<D, BF>), dim3(a.B * a.Hq), dim3(256), 0, s, a);
 }
 
@@ -996,7 +1017,8 @@ extern "C" {
 size_t kq_sdpa_workspace_bytes(int32_t B, int32_t Hq, int32_t Hkv, int32_t D, int32_t max_len) {
     if (B <= 0 || Hkv <= 0 || Hq <= 0 || Hq % Hkv || D <= 0) return 0;
     // one sizer for both caches: the larger of their plans
-    const size_t a = ws_bytes(B, Hq, Hkv, D, max_len, false), b = ws_bytes(B, Hq, Hkv, D, max_len, true);
+    const size_t a = ws_layout(B, Hq, Hkv, D, max_len, false).bytes();
+    const size_t b = ws_layout(B, Hq, Hkv, D, max_len, true).bytes();
     return a > b ? a : b;
 }
 
@@ -1059,8 +1081,8 @@ int ragged_impl(const void *q, const void *k, const void *v, const Q8Scales *q8,
     if (((uintptr_t)q & 15) || ((uintptr_t)k & kv_align) || ((uintptr_t)v & kv_align) || ((uintptr_t)out & 15))
         return KQ_ERR_BAD_ALIGN;
     WsLayout w = ws_layout(B, Hq, Hkv, D, max_len, q8 != nullptr);
-    if (workspace_bytes < w.part_bytes + w.ml_bytes) w = ws_layout(B, Hq, Hkv, D, max_len, q8 != nullptr, true);
-    if (!workspace || workspace_bytes < w.part_bytes + w.ml_bytes) return KQ_ERR_WORKSPACE_TOO_SMALL;
+    if (workspace_bytes < w.bytes()) w = ws_layout(B, Hq, Hkv, D, max_len, q8 != nullptr, true);
+    if (!workspace || workspace_bytes < w.bytes()) return KQ_ERR_WORKSPACE_TOO_SMALL;
     SdpaArgs a;
     a.q = (const uint16_t *)q;
     a.k = (const uint16_t *)k;
@@ -1084,15 +1106,18 @@ int ragged_impl(const void *q, const void *k, const void *v, const Q8Scales *q8,
     a.Hq = Hq;
     a.Hkv = Hkv;
     a.G = Hq / Hkv;
-    a.split = w.split;
-    a.max_splits = max_len <= 0 ? 1 : (max_len + a.split - 1) / a.split;
+    a.rule = w.rule;
+    a.split = 0;
+    a.max_splits = w.max_splits;
     a.max_len = max_len;
     a.scale_log2 = scale * 1.4426950408889634f;
-    // one wave per unit; the unit count is bounded by B * Hkv * max_splits
-    // (rows are shorter on the device side), extra waves exit at once
-    const int64_t upper = (int64_t)B * Hkv * a.max_splits;
-    const int grid = (int)(upper < (1 << 22) ? upper : (1 << 22));
+    // one wave per unit of rows of max_len (shorter ones leave waves that exit
+    // at once); a row just below a line of the split rule has up to twice as
+    // many splits of half the length, and its waves take two
+    const int row_waves = row_splits(a.rule, max_len);
+    const int64_t upper = (int64_t)B * Hkv * row_waves;
     a.direct = pad && upper < (1 << 22) && Hkv < (1 << 16) && B < (1 << 16);
+    const int grid = a.direct ? row_waves : (int)(upper < (1 << 22) ? upper : (1 << 22));
     const bool merge = a.max_splits > 1;
     hipStream_t s = (hipStream_t)stream;
     const bool bf = dtype == KQ_DTYPE_BF16;
@@ -1257,6 +1282,7 @@ int cascade_impl(const void *q, const void *k_shared, const void *v_shared, cons
     a.Hkv = Hkv;
     a.G = Hq / Hkv;
     const CascadePlan plan = cascade_plan(P, S, rows, Hkv, a.G, D);
+    a.rule = SplitRule{};
     a.split = plan.split2;
     a.split1 = plan.split1;
     a.n1 = (P + a.split1 - 1) / a.split1;
@@ -1365,8 +1391,7 @@ extern "C" int kq_sdpa_decode_gqa_noalloc(const void *q, const void *k, const vo
                                           kq_stream_t stream) {
     if (B == 0) return KQ_OK;
     if (B < 0 || Hq <= 0 || Hkv <= 0 || Hq % Hkv || D <= 0 || L < 0) return KQ_ERR_BAD_SHAPE;
-    const size_t need = ws_bytes(B, Hq, Hkv, D, L, false);
-    if (need > KQ_SDPA_NOALLOC_SCRATCH_BYTES) return KQ_ERR_WORKSPACE_TOO_SMALL;
+    if (ws_layout(B, Hq, Hkv, D, L, false, true).bytes() > KQ_SDPA_NOALLOC_SCRATCH_BYTES) return KQ_ERR_WORKSPACE_TOO_SMALL;
     void *ws = nullptr;
     if (const int rc = scratch_ptr(&ws)) return rc;
     const PaddedKv pad{batch_stride, head_stride, starts};

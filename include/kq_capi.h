@@ -326,9 +326,18 @@ int kq_moe_router_topk(const void *logits, int logits_dtype, int64_t logits_row_
                        float *scores, kq_stream_t stream);
 
 /* ---- ragged GQA decode attention ----------------------------------------- */
-/* Workspace of kq_sdpa_decode_ragged: fp32 split partials (O, m, l) for
- * B * Hkv * ceil(max_len / split) splits; no zero-fill needed.  Calls that
- * share a workspace must be ordered (same stream).
+/* Workspace of kq_sdpa_decode_ragged: fp32 split partials (O, m, l), as many
+ * splits per (row, kv head) as a row of at most max_len keys can have; no
+ * zero-fill needed.  A buffer of at least B * Hq * ceil(max_len / 512) * (D + 2)
+ * floats (the first D of each rounded up together to 256 bytes) is served too,
+ * with splits of 512 or 1024 tokens.  Calls that share a
+ * workspace must be ordered (same stream).
+ *
+ * A row's split lengths follow from its own keys, the head counts, D and the
+ * cache's type, not from the other rows: its output is bitwise that of a call
+ * on the row alone.  Two plans are for the launch instead: 1024 tokens for
+ * every row once B * Hkv * ceil(max_len / 1024) reaches 8 waves per CU, and
+ * that of a workspace smaller than this size.
  *
  * ragged_decode_attention(q, k, v, pads, scale) (gmlx/qwen35_attn.py:395-493)
  * and kq.sdpa_decode_gqa(q, k, v, scale, starts=) (gmlx/gemma4_batched_sdpa.py:
@@ -385,9 +394,10 @@ int kq_sdpa_decode_gqa(const void *q, const void *k, const void *v, int64_t batc
  * memory (code under HIP graph capture, tight serving loops, harnesses that
  * forbid hipMalloc).  The split partials live in a device array the library
  * holds on each GPU it runs on (KQ_SDPA_NOALLOC_SCRATCH_BYTES, until the
- * process ends); calls needing more (kq_sdpa_workspace_bytes(B, Hq, Hkv, D,
- * L) above the limit) return KQ_ERR_WORKSPACE_TOO_SMALL and launch nothing.
- * Same outputs as kq_sdpa_decode_gqa (the same kernels and split plan).  All
+ * process ends); calls whose long splits need more (B * Hq * ceil(L /
+ * 512) * (D + 2) floats, half of that where 1024-token splits apply) return
+ * KQ_ERR_WORKSPACE_TOO_SMALL and launch nothing.  Same outputs as
+ * kq_sdpa_decode_gqa given a workspace of the array's size.  All
  * calls on one GPU share the array: calls that overlap there (other streams
  * or threads) race; order them. */
 #define KQ_SDPA_NOALLOC_SCRATCH_BYTES ((size_t)32 << 20)

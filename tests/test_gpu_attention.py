@@ -240,9 +240,10 @@ def test_batch_row_equals_single_row(split, dtype_name, monkeypatch):
     one plan for the batch and for each row, no drift at all).  Covered:
     ragged_decode_attention on [B, Hkv, L, D] with the reference's live pads
     (:97), sdpa_decode_gqa with device starts over the 16-bit and the 8-bit
-    affine cache, and the per-row slab layout.  Splits run 512 or 1024 tokens
-    by the launch's size, so the batched and the single-row call are also
-    compared with the split forced either way."""
+    affine cache, and the per-row slab layout.  Split lengths follow from the
+    row alone, but run 1024 tokens in the largest launches, so the batched and
+    the single-row call are also compared with the split forced to 512 and to
+    1024."""
     import torch
     from gmlx_amd import ops
     from helpers import q8_affine
