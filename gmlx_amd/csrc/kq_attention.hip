@@ -725,6 +725,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(D <= 128 ? 2
     __shared__ __attribute__((aligned(16))) uint8_t qs[q_in_lds<D, Q8>() ? q_lds_bytes<D>() : 16];
     const uint32_t q_lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void *)qs;
     const int r = kq_lane() & 15;
+    const int direct_splits = a.direct ? row_unit_splits(a, blockIdx.z) : 0;
     for (int u = blockIdx.x;; u += gridDim.x) {
         int b, h, s;
         if (a.direct) {
@@ -732,7 +733,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(D <= 128 ? 2
             s = u;
             h = blockIdx.y;
             b = blockIdx.z;
-            if (s >= row_unit_splits(a, b)) return;
+            if (s >= direct_splits) return;
         } else if (!map_unit(a, u, b, h, s)) {
             return;
         }
