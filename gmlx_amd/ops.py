@@ -125,9 +125,11 @@ class _Workspaces:
         if cur is None or cur.numel() < nbytes:
             if cur is not None:
                 self._retired.append(cur)
-            # powers of two: a decode loop whose partials grow by one split at
-            # a time replaces (and retires) its buffer a few times, not each
-            size = 1 << (max(nbytes, 1 << 16) - 1).bit_length()
+            size = max(nbytes, 1 << 16)
+            if kind.startswith("sdpa"):
+                # powers of two: a decode loop whose partials grow by one split at
+                # a time replaces (and retires) its buffer a few times, not each
+                size = 1 << (size - 1).bit_length()
             cur = torch.zeros(size, dtype=torch.uint8, device=device)
             self._ws[key] = cur
         return cur

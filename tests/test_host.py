@@ -343,3 +343,19 @@ def test_inline_assembly_declares_its_use_of_m0():
             writes = re.search(r"\bs_\w+\s+m0\b", code)
             assert ('"m0"' in operands) if writes else ('"{m0}"' in operands), (name, stmt)
     assert found  # kq_gemm.hip's copies
+
+
+def test_workspaces_take_what_is_needed():
+    """Matmul and gather workspaces (a prompt's prepared rows and partials may
+    take gigabytes) are as large as asked; attention's, which grow by a split at
+    a time, go by powers of two.  A buffer is kept while it is large enough, and
+    a replaced one is not freed."""
+    from gmlx_amd import ops
+    ws, dev = ops._Workspaces(), torch.device("cpu")
+    for kind, want in (("matmul", 3 << 20), ("gather", 3 << 20), ("mlp", 3 << 20), ("sdpa", 4 << 20),
+                       ("sdpa_cascade", 4 << 20)):
+        assert ws.get(kind, dev, 0, 100).numel() == 1 << 16
+        buf = ws.get(kind, dev, 0, 3 << 20)
+        assert buf.numel() == want, kind
+        assert ws.get(kind, dev, 0, 2 << 20) is buf and not buf.any()
+    assert len(ws._retired) == 5
