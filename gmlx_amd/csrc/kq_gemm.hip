@@ -836,6 +836,10 @@ int launch_gather(const KqGemmGather &a, int grid, hipStream_t s) {
 
 int tile_cols(int mt, bool glu) { return (mt == 4 ? 256 : 128) / (glu ? 2 : 1); }
 
+// Workgroups a launch may have: its threads are counted in 32 bits, and the
+// grid is rounded up to the eight XCDs.
+int64_t max_groups(int mt) { return (((int64_t)1 << 32) - 1) / (mt == 4 ? 512 : 256) - 8; }
+
 // Tile height and K slices of a dense launch.
 struct Plan {
     int mt, slices, tiles;
@@ -881,7 +885,7 @@ Plan make_plan(const kq_matmul_problem *ps, int n, bool glu) {
         for (int s = 1; s <= 8; ++s) {
             if (forced_s && s != forced_s && !glu) continue;
             if (s > 1 && (glu || nb_min < 4 * s || tiles > (int64_t)(KQ_MATMUL_COUNTER_BYTES / 4))) break;
-            if (tiles * s > (1 << 28)) break;
+            if (tiles * s > max_groups(mt)) break;
             const int64_t part = s > 1 ? tiles * s * (mt * 16 * (mt == 4 ? 8 : 4) * 64 * 4) : 0;
             const double us = ((double)nb_max / s + 1.5) * stage_us(mt, codec, (double)tiles * s, cus) +
                               (s > 1 ? 4.0 + 2e-6 * (double)part / 3.0 : 0.0);
@@ -1050,20 +1054,23 @@ static bool gather_pays(const KqGemmGather &a, bool streams) {
     return theirs > 1.08 * tiles;
 }
 
+// Workgroups of a gather: they bound every chunk of every segment.
+static int64_t gather_groups(const KqGemmGather &a, int mt) {
+    const int slots = a.n_experts < a.n_pairs ? a.n_experts : a.n_pairs, cols = tile_cols(mt, a.w1 != nullptr);
+    return ((int64_t)a.n_pairs / (32 * mt) + slots) * ((a.N + cols - 1) / cols);
+}
+
 bool kq_gemm_gather_eligible(const KqGemmGather &a, int64_t x_rows, int64_t x_row_stride, bool streams) {
     const int mode = env_int("GMLX_KQ_GEMM", 1);
-    return mode != 0 && addressable(x_rows, x_row_stride) && (mode == 2 || gather_pays(a, streams));
+    const int mt = gather_mt(a.n_pairs, a.n_experts < a.n_pairs ? a.n_experts : a.n_pairs);
+    return mode != 0 && addressable(x_rows, x_row_stride) && gather_groups(a, mt) <= max_groups(mt) &&
+           (mode == 2 || gather_pays(a, streams));
 }
 
 int kq_gemm_gather_launch(const KqGemmGather &a, hipStream_t s) {
     const bool glu = a.w1 != nullptr;
-    // the grid bounds every chunk of every segment
-    const int slots = a.n_experts < a.n_pairs ? a.n_experts : a.n_pairs;
-    const int mt = gather_mt(a.n_pairs, slots);
-    const int64_t chunks = (int64_t)a.n_pairs / (32 * mt) + slots;
-    const int64_t n_tiles = (a.N + tile_cols(mt, glu) - 1) / tile_cols(mt, glu);
-    if (chunks * n_tiles > (1 << 28)) return KQ_ERR_BAD_SHAPE;
-    const int grid = 8 * (int)((chunks * n_tiles + 7) / 8);
+    const int mt = gather_mt(a.n_pairs, a.n_experts < a.n_pairs ? a.n_experts : a.n_pairs);
+    const int grid = 8 * (int)((gather_groups(a, mt) + 7) / 8);
     if (mt == 2) return glu ? launch_gather<2, 4, true>(a, grid, s) : launch_gather<2, 4, false>(a, grid, s);
     return glu ? launch_gather<1, 4, true>(a, grid, s) : launch_gather<1, 4, false>(a, grid, s);
 }

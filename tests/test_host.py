@@ -359,3 +359,18 @@ def test_workspaces_take_what_is_needed():
         assert buf.numel() == want, kind
         assert ws.get(kind, dev, 0, 2 << 20) is buf and not buf.any()
     assert len(ws._retired) == 5
+
+
+def test_glu_launch_stays_within_the_grid():
+    """kq_glu_matmul declines (callers run the two steps) a problem whose tiles
+    would take 2^32 threads or more, the most a launch can have, and takes one of
+    half its columns: bf16 rows without a workspace then get as far as that."""
+    from gmlx_amd import _lib
+    L = _lib.lib()
+    M, K, p = 4190000, 256, 1 << 20  # rows within 2 GiB; the pointers are never read
+
+    def call(I):
+        return L.kq_glu_matmul(p, _lib.DTYPE_BF16, K, M, K, p, p, 144, 12, I, 0, p, _lib.DTYPE_BF16, I, None, 0, None)
+
+    assert call(32768) == _lib.KQ_ERR_WORKSPACE_TOO_SMALL
+    assert call(65536) == _lib.KQ_ERR_BAD_SHAPE
