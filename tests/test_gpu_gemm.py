@@ -130,46 +130,127 @@ def test_dense_glu(M, I, codec, act, mt, dtype_name, monkeypatch):
     assert ops._glu_matmul(x[:64], _dev(gw), _dev(uw), codec, act, ops._stream(x)) is None
 
 
+@pytest.mark.parametrize("dtype_name", ["float16", "bfloat16", "float32"])
 @pytest.mark.parametrize("mt", ["1", "2"])
 @pytest.mark.parametrize("codec", CODECS)
-def test_long_segments(codec, mt, monkeypatch):
+def test_long_segments(codec, mt, dtype_name, monkeypatch):
     """Gathers whose segments are longer than a tile, one row, empty and out of
-    range: plain with a bias, clamped GLU with biases, and the shared-expert
-    layout's spare rows, against the per-tile gathers (GMLX_KQ_GEMM=0) and
-    fp64."""
+    range: plain with a bias, clamped GLU with biases, the shared-expert
+    layout's spare rows and the down gather over them, against the small-batch
+    gathers (GMLX_KQ_GEMM=0) and fp64.  bf16 and fp32 rows are 2^-20 to 2^20 in
+    size, and every pair row is held to its own largest value."""
     import torch
     from gmlx_amd import ops
     rng = np.random.default_rng(11)
-    E, T, k, D, I = 5, 150, 2, 512, 200
+    E, T, k, D, I = 5, 150, 2, 768, 200
     idx = np.full((T, k), 1)
     idx[:, 1] = rng.integers(2, 4, T)
     idx[7] = [0, 5]      # one row for expert 0, an id out of range; expert 4 empty
     idx[149, 1] = -1
     w = np.stack([_wire(rng, codec, I, D) for _ in range(E)])
     wu = np.stack([_wire(rng, codec, I, D) for _ in range(E)])
-    x = fp16_rows(rng, T, D)
+    wd = np.stack([_wire(rng, codec, 130, 256) for _ in range(E)])
+    x, hid = fp16_rows(rng, T, D).astype(np.float32), fp16_rows(rng, T * (k + 1), 256).astype(np.float32)
+    xc = x
+    if dtype_name != "float16":
+        size = np.exp2(rng.integers(-20, 21, (T, 1))).astype(np.float32)
+        # (the clamps bound h: against large gates its fp32 error has no bound relative to the row)
+        x, xc = x * size, x * np.minimum(size, 1)
+        hid *= np.exp2(rng.integers(-20, 21, (T * (k + 1), 1))).astype(np.float32)
+    dt = getattr(torch, dtype_name)
     b0, b1 = (rng.normal(0, 1, (E, I)).astype(np.float32) for _ in range(2))
-    xd, idxd, wd, wud, b0d, b1d = (_dev(a) for a in (x, idx.astype(np.int32), w, wu, b0, b1))
-    sg, su = wd[0].contiguous(), wud[0].contiguous()
+    idxd, wgd, wud, wdd, b0d, b1d = (_dev(a) for a in (idx.astype(np.int32), w, wu, wd, b0, b1))
+    xd, xcd, hd = _dev(x).to(dt), _dev(xc).to(dt), _dev(hid).to(dt).reshape(T, k + 1, 256)
+    sg, su, sd = wgd[0].contiguous(), wud[0].contiguous(), wdd[0].contiguous()
+    ones = torch.zeros(T, k + 1, device="cuda")
 
     def run(mode):
         monkeypatch.setenv("GMLX_KQ_GEMM", mode)
         monkeypatch.setenv("GMLX_KQ_GEMM_MT", mt)
-        y = ops.gather_qmm(xd, wd, None, codec, indices=idxd, out_dtype=torch.float32, bias=b0d)
-        h = ops.moe_glu_gather_kq(xd, wd, wud, codec, idxd, act="swiglu_clamp", gate_bias=b0d, up_bias=b1d)
-        hs = ops.moe_glu_gather_shexp_kq(xd, wd, wud, sg, su, codec, idxd)
-        return y.cpu().numpy(), h.cpu().numpy(), hs.cpu().numpy()
+        y = ops.gather_qmm(xd, wgd, None, codec, indices=idxd, out_dtype=torch.float32, bias=b0d).reshape(T, k, I)
+        h = ops.moe_glu_gather_kq(xcd, wgd, wud, codec, idxd, act="swiglu_clamp", gate_bias=b0d, up_bias=b1d)
+        hs = ops.moe_glu_gather_shexp_kq(xd, wgd, wud, sg, su, codec, idxd)
+        dn = []
+        for s in range(k + 1):  # the mix with one weight of 1: slot s alone
+            one = ones.clone()
+            one[:, s] = 1
+            dn.append(ops.gather_qmv_mix_kq(hd, wdd, sd, codec, idxd, one))
+        return [t.cpu().numpy() for t in (y, h, hs, torch.stack(dn, 1))]
+
+    def rows_rel(a, b):
+        a, b = (t.reshape(-1, t.shape[-1]).astype(np.float64) for t in (a, b))
+        big = np.abs(b).max(1)
+        assert not a[big == 0].any()
+        return (np.abs(a - b).max(1)[big > 0] / big[big > 0]).max()
 
     old, new = run("0"), run("2")
     for a, b in zip(new, old):
-        assert okq.max_rel(a, b) <= 2e-6 * 16  # fp32 sums in another order
-    ref = np.zeros((T, k, I))
+        assert rows_rel(a, b) <= 2e-6 * 16  # fp32 sums in another order
+    xf, hf = xd.double().cpu().numpy(), hd.double().cpu().numpy()
+    W, Wd = (okq.dequantize(t, codec).astype(np.float64) for t in (w, wd))
+    ref, refd = np.zeros((T, k, I)), np.zeros((T, k + 1, 130))
     for t in range(T):
         for s in range(k):
             e = idx[t, s]
             if 0 <= e < E:
-                ref[t, s] = okq.qmm_ref(x[t:t + 1], w[e], codec)[0] + b0[e]
-    assert okq.max_rel(new[0][:, :, 0], ref) <= _tol(codec)
+                ref[t, s] = W[e] @ xf[t] + b0[e]
+                refd[t, s] = Wd[e] @ hf[t, s]
+        refd[t, k] = Wd[0] @ hf[t, k]
+    # (fp32 rows enter rounded to 11 bits)
+    tol = TOL if dtype_name == "float32" else _tol(codec)
+    assert rows_rel(new[0], ref) <= tol
+    assert rows_rel(new[3], refd) <= tol
+
+
+@pytest.mark.parametrize("codec", CODECS)
+def test_more_segments_than_a_wave(codec, monkeypatch):
+    """130 experts, a third of them empty, segments of one row to four tiles: the
+    chunk table runs over three rounds of 64 segments.  Plain, GLU and per-pair
+    gathers of bf16 rows against fp64."""
+    import torch
+    from gmlx_amd import ops
+    monkeypatch.setenv("GMLX_KQ_GEMM", "2")
+    monkeypatch.setenv("GMLX_KQ_GEMM_MT", "1")
+    rng = np.random.default_rng(130)
+    E, N, K = 130, 72, 256
+    counts = rng.integers(1, 6, E)
+    counts[rng.random(E) < 1 / 3] = 0
+    counts[[3, 63, 64, 65, 128, 129]] = [100, 33, 0, 32, 70, 1]
+    ids = rng.permutation(np.repeat(np.arange(E), counts))
+    k = 2
+    idx = ids[:len(ids) // k * k].reshape(-1, k)
+    T = len(idx)
+    w, wu = (np.stack([_wire(rng, codec, N, K) for _ in range(E)]) for _ in range(2))
+    W, U = (okq.dequantize(t, codec).astype(np.float64) for t in (w, wu))
+    xd = _dev(fp16_rows(rng, T, K)).bfloat16()
+    hd = _dev(fp16_rows(rng, T * k, K)).bfloat16().reshape(T, k, K)
+    idxd, wd, wud = _dev(idx.astype(np.int32)), _dev(w), _dev(wu)
+    y = ops.gather_qmm(xd, wd, None, codec, indices=idxd, out_dtype=torch.float32).reshape(T, k, N).cpu().numpy()
+    h = ops.moe_glu_gather_kq(xd, wd, wud, codec, idxd).cpu().numpy()
+    p = ops.gather_qmv_kq(hd, wd, codec, idxd).cpu().numpy()
+    xf, hf = xd.double().cpu().numpy(), hd.double().cpu().numpy()
+    g, u = (np.einsum("tknj,tj->tkn", M[idx], xf) for M in (W, U))
+    assert okq.max_rel(y, g) <= _tol(codec)
+    assert okq.max_rel(h, 0.5 * g * (1 + np.tanh(0.5 * g)) * u) <= TOL
+    assert okq.max_rel(p, np.einsum("tknj,tkj->tkn", W[idx], hf)) <= _tol(codec)
+
+
+@pytest.mark.parametrize("codec", CODECS)
+def test_dense_kernel_past_64_rows(codec, monkeypatch):
+    """The dense kernel over more than one chunk of 64 rows (GMLX_KQ_GEMM=0), and
+    where a group of a longer and a shorter problem takes it by itself."""
+    import torch
+    from gmlx_amd import ops
+    rng = np.random.default_rng(64)
+    K = 1024
+    x, (w, v) = fp16_rows(rng, 150, K), (_wire(rng, codec, n, K) for n in (40, 77))
+    xd = _dev(x)
+    a, b = ops.quantized_matmul_grouped([(xd, _dev(w), codec), (xd[:20], _dev(v), codec)], out_dtype=torch.float32)
+    monkeypatch.setenv("GMLX_KQ_GEMM", "0")
+    c = ops.quantized_matmul(xd, _dev(w), None, codec, out_dtype=torch.float32)
+    assert torch.equal(a, c)
+    assert okq.max_rel(c.cpu().numpy(), okq.qmm_ref(x, w, codec)) <= TOL
+    assert okq.max_rel(b.cpu().numpy(), okq.qmm_ref(x[:20], v, codec)) <= TOL
 
 
 @pytest.mark.parametrize("T,tiles", [(9, False), (33, False), (512, True)])

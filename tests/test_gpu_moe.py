@@ -66,9 +66,12 @@ def test_gather_qmm(codec):
     assert okq.max_rel(got.float().cpu().numpy()[:, :, 0], ref) <= TOL
 
 
-def test_gather_many_rows_per_expert():
-    """Segments larger than one 64-row chunk (prefill-sized)."""
+@pytest.mark.parametrize("gemm", ["0", "2"])
+def test_gather_many_rows_per_expert(gemm, monkeypatch):
+    """Segments larger than one 64-row chunk (prefill-sized), on the per-tile
+    gathers and on the matrix-core tiles."""
     from gmlx_amd import ops
+    monkeypatch.setenv("GMLX_KQ_GEMM", gemm)
     rng = np.random.default_rng(2)
     E, N, K, T, k = 3, 48, 256, 150, 2
     w = _experts(rng, "q4_k", E, N, K)
@@ -127,9 +130,10 @@ def test_moe_glu_then_down_then_mix(act):
     ("q6_k", "iq2_xxs", 3072, 512, 8, 5, 8),     # K = 12 super-blocks; every expert touched
 ])
 def test_streaming_gather_matches_tile_gather(gcodec, dcodec, D, I, E, T, k, monkeypatch):
-    """The streaming gather (every form forced, GMLX_KQ_SGATHER=2) against
-    the per-tile gather kernels (=0) and the fp64 oracle: the GLU gather then
-    the per-pair down gather, with one never-routed pair (zeros)."""
+    """The streaming gather (every form forced, GMLX_KQ_SGATHER=2), the per-tile
+    gather kernels (=0), both without the matrix-core tiles (GMLX_KQ_GEMM=0),
+    and those tiles (=2) against the fp64 oracle: the GLU gather then the
+    per-pair down gather, with one never-routed pair (zeros)."""
     from gmlx_amd import ops
     rng = np.random.default_rng(D + I + E)
     gw = _experts(rng, gcodec, E, I, D)
@@ -139,7 +143,8 @@ def test_streaming_gather_matches_tile_gather(gcodec, dcodec, D, I, E, T, k, mon
     idx = np.stack([rng.choice(E, size=k, replace=False) for _ in range(T)]).astype(np.int32)
     idx[-1, 0] = E + 3  # never routed
     outs = {}
-    for mode in ("stream", "tile"):
+    for mode in ("stream", "tile", "gemm"):
+        monkeypatch.setenv("GMLX_KQ_GEMM", "2" if mode == "gemm" else "0")
         monkeypatch.setenv("GMLX_KQ_SGATHER", "2" if mode == "stream" else "0")
         h = ops.moe_glu_gather_kq(_dev(x), _dev(gw), _dev(uw), gcodec, _dev(idx))
         y = ops.gather_qmv_kq(h, _dev(dw), dcodec, _dev(idx))
@@ -162,6 +167,7 @@ def test_streaming_gather_matches_tile_gather(gcodec, dcodec, D, I, E, T, k, mon
                          for t in range(T)])
         assert okq.max_rel(y, yref) <= TOL, (mode, okq.max_rel(y, yref))
     assert okq.max_rel(outs["stream"][0], outs["tile"][0]) <= TOL
+    assert okq.max_rel(outs["gemm"][0], outs["tile"][0]) <= TOL
 
 
 def test_router_topk_matches_numpy():
@@ -206,15 +212,18 @@ def test_switch_linear_module():
     assert okq.max_rel(got[:, :, 0], ref) <= TOL
 
 
-@pytest.mark.parametrize("codec,scodec,T,k,E", [("q4_k", None, 5, 4, 16), ("q4_k", "q6_k", 3, 8, 64),
-                                                  ("iq2_xxs", None, 8, 8, 32), ("q6_k", "q4_k", 1, 2, 4)])
-def test_shared_expert_glu_and_mix(codec, scodec, T, k, E):
+@pytest.mark.parametrize("codec,scodec,T,k,E,gemm", [
+    ("q4_k", None, 5, 4, 16, "1"), ("q4_k", "q6_k", 3, 8, 64, "1"), ("iq2_xxs", None, 8, 8, 32, "1"),
+    ("q6_k", "q4_k", 1, 2, 4, "1"), ("q4_k", "q6_k", 9, 4, 16, "1"), ("iq2_xxs", None, 33, 2, 8, "1"),
+    ("q4_k", "q6_k", 9, 4, 16, "2"), ("iq2_xxs", None, 33, 2, 8, "2"), ("q6_k", "q4_k", 70, 2, 4, "2")])
+def test_shared_expert_glu_and_mix(codec, scodec, T, k, E, gemm, monkeypatch):
     """moe_glu_gather_shexp_kq / gather_qmv_mix_kq: the shared expert in slot
     k of h and of the mix (gmlx/modules.py:571-584, 777-787), a different
     codec for the shared matrices included; routed slots equal the plain
-    fused ops' results."""
+    fused ops' results.  gemm "2": on the matrix-core tiles."""
     import torch
     from gmlx_amd import ops
+    monkeypatch.setenv("GMLX_KQ_GEMM", gemm)
     rng = np.random.default_rng(T * 100 + k)
     D, I = 512, 256
     sc_codec = scodec or codec
@@ -485,13 +494,16 @@ def test_kquant_embedding(codec, dtype_name):
     ("q4_k", 3, 2, 4, 4096, 64, True),        # 16 super-blocks per row: the split-K gather
 ])
 @pytest.mark.parametrize("hdt", ["float32", "float16"])
-def test_down_gather_with_mix_equals_two_steps(dcodec, T, k, E, I, N, bad, hdt):
+@pytest.mark.parametrize("gemm", ["0", "2"])
+def test_down_gather_with_mix_equals_two_steps(dcodec, T, k, E, I, N, bad, hdt, gemm, monkeypatch):
     """gather_qmv_mix_ns_kq bitwise equal to the per-pair gather followed by
     the slot-ordered fp32 mix written out in torch; repeated calls and graph
     replays bitwise equal; and within tolerance of fp64
-    (gmlx/modules.py:591-593)."""
+    (gmlx/modules.py:591-593).  On the small-batch gathers and, gemm "2", on
+    the matrix-core tiles."""
     import torch
     from gmlx_amd import ops
+    monkeypatch.setenv("GMLX_KQ_GEMM", gemm)
     rng = np.random.default_rng(T * 31 + k + E + I)
     dw = _dev(_experts(rng, dcodec, E, N, I))
     idx_np = np.stack([rng.choice(E, size=k, replace=False) for _ in range(T)]).astype(np.int32)
