@@ -13,7 +13,8 @@
 //  - Activations do: one super-block (BM rows x 512 bytes) per stage in two
 //    LDS buffers, copied by direct-to-LDS loads one stage ahead; every
 //    wave reads the same rows, 1 KB per v_mfma_f32_32x32x16_f16.
-//  - The B operand is the exact integer code of kq_mma.h; each super-block
+//  - The B operand is the integer code of kq_mma.h (exact; Q6_K's products
+//    above 2048 round to 11 bits there as here); each super-block
 //    runs as its own MFMA chain P and folds into the accumulators with the
 //    block's fp32 factor.  Q4_K's minimum term multiplies fp32 sub-block sums
 //    of the activations, held as three bf16 parts (24 bits), by the integer
@@ -23,9 +24,10 @@
 //
 // Bound by the matrix cores and the decode that shares the SIMDs with them.
 // Measured against the small-batch dense kernel and the per-tile gathers: an
-// MLP of 2048 bf16 rows (4096 x 12288, Q4_K / Q6_K) 3911 -> 849 us, 725
-// TFLOP/s; the projections of a layer of 333 fp16 rows 832 -> 295 us; an MoE
-// layer of 500 bf16 tokens (128 experts of 2048 x 768, 8 a token) 479 -> 291.
+// MLP of 2048 bf16 rows (4096 x 12288, Q4_K / Q6_K) 3902 -> 876 us, 706
+// TFLOP/s (841 to 881 us over the boxes it ran on); the projections of a layer
+// of 333 fp16 rows 830 -> 298 us; an MoE layer of 500 bf16 tokens (128 experts
+// of 2048 x 768, 8 a token) 480 -> 294.
 //
 // Lane l = 32 h + r.  Operand layouts of v_mfma_f32_32x32x16: A row / B column
 // r, k values 8 h .. 8 h + 7; result element i: row 8 (i / 4) + 4 h + i % 4,

@@ -106,7 +106,10 @@ typedef struct {
  * zero them once when the buffer is allocated (any fill); each call leaves
  * them zero, and nothing else may write them (do not hand such a workspace
  * to the attention entry points).  Calls sharing a workspace must be
- * ordered (same stream). */
+ * ordered (same stream).  A captured call keeps the workspace it was captured
+ * with: replays of graphs that share one run one at a time, and not beside
+ * other calls on it.  That holds wherever kq_matmul_workspace_bytes or
+ * kq_gather_workspace_bytes is not 0, for fp16 activations as well. */
 #define KQ_MATMUL_COUNTER_BYTES ((size_t)16 << 10)
 
 /* Workspace bytes kq_quantized_matmul_grouped needs for these problems and
