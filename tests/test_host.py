@@ -4,6 +4,8 @@ the ops' CPU-side validation and decline rails, fault injection, the wire-K
 rule, and the leaf-module swap."""
 import os
 import re
+import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -374,3 +376,10 @@ def test_glu_launch_stays_within_the_grid():
 
     assert call(32768) == _lib.KQ_ERR_WORKSPACE_TOO_SMALL
     assert call(65536) == _lib.KQ_ERR_BAD_SHAPE
+
+
+def test_nn_is_an_attribute_of_the_package():
+    """gmlx_amd.nn without an import of its own, in a fresh interpreter."""
+    r = subprocess.run([sys.executable, "-c", "import gmlx_amd; print(gmlx_amd.nn.KQuantLinear.__name__)"],
+                       cwd=ROOT, capture_output=True, text=True)
+    assert r.returncode == 0 and r.stdout.strip() == "KQuantLinear", r.stderr[-500:]
