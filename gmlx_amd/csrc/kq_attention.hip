@@ -921,13 +921,17 @@ int env_int(const char *name, int dflt) {
 //   1 of 32768      37.0 / 28.6 / 24.7 / 33.1     3 rows  74.9 / 64.0 / 58.2 / 56.7
 // and at D = 256, two query heads
 //   1 row of 1600   12.5 / 14.4 / 20.8 / 33.6    32 rows  93.8 / 92.4 / 90.1 / 84.7
-// So: up to 256 tokens one split (no merge; 512 past four query heads a kv
-// head, whose merges cost as many times more; 128 at D = 256, none past it or
-// there in 8 bits); then 64, 128 and 256 up to the lines below, past them 512.
-// Against 512 throughout, 376 launches of 1 to 32 equal rows took 0.66 times
-// as long in the geometric mean; 47 took over 3 % longer, 46 of them by at
-// most 13 % and 32 rows of 400 tokens 19 us against 14.5: there the merge
-// costs more than the shorter chain gives, and with one row it is 8 against 12.
+// So: short rows one split, with no merge (256 tokens; 512 past eight query
+// heads a kv head, whose merges cost as many times more; 64 in 8 bits, 256
+// past eight; 128 at D = 256); then 64, 128 and 256 up to the lines below,
+// past them 512.  A longer one-split line would cost mixed batches, which wait
+// for their longest chain: three rows of 391, 771 and 1733 tokens 92 us over
+// eight layers, 137 with it at 512.  Against 512 throughout, 526 launches of 1
+// to 32 equal rows took 0.71 times as long in the geometric mean; 65 took over
+// 3 % longer: 32 rows of 300 to 500 tokens by up to 1.45 times (16 us against
+// 12 with four query heads a kv head, where one row takes 8 against 10), 32 of
+// 100 in 8 bits by up to 1.35 (not past eight query heads), the others by at
+// most 17 %, nearly all of them 32 rows.
 // A launch of B * Hkv * ceil(max_len / 1024) >= 8 waves a CU takes 1024 for
 // every row (C3: 353 against 372 us at 512): a row's bits there are not those
 // of the row alone.  `wide` keeps to 512 and 1024: the plan
@@ -943,8 +947,9 @@ SplitRule split_rule(int B, int Hq, int Hkv, int D, int max_len, bool q8, bool w
         r.rest = 1024;
     } else if (!wide) {
         if (D > 128) r = SplitRule{q8 || D > 256 ? 0 : 128, 1024, 8192, 32768, 512};
-        else if (q8) r = SplitRule{256, 1024, 2048, 32768, 512};
-        else r = Hq > 4 * Hkv ? SplitRule{512, 0, 1024, 8192, 512} : SplitRule{256, 512, 4096, 8192, 512};
+        else if (q8) r = SplitRule{Hq > 8 * Hkv ? 256 : 0, 1024, 2048, 32768, 512};
+        else if (Hq > 8 * Hkv) r = SplitRule{512, 0, 1024, 8192, 512};
+        else r = SplitRule{256, 512, Hq > 4 * Hkv ? 1024 : 4096, 8192, 512};
     }
     return r;
 }

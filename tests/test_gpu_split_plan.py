@@ -15,12 +15,12 @@ def _rows(rng, torch, B, Hq, Hkv, L, D, dt):
     return mk(B, Hq, 1, D), mk(B, Hkv, L, D), mk(B, Hkv, L, D)
 
 
-# rows of L and L - 1 keys on both sides of each line: 256, 512, 4096 (1024 past four
-# query heads a kv head) and 8192 up to head dim 128; 128, 1024, 8192 and 32768
+# rows of L and L - 1 keys on both sides of each line: 256 (512 past eight query heads
+# a kv head), 512, 4096 (1024 past four) and 8192 up to head dim 128; 128, 1024, 8192 and 32768
 # past it; and 2048 waves of 1024 tokens
 @pytest.mark.parametrize("B,Hq,Hkv,L,D,dtype_name", [
     (3, 8, 2, 257, 64, "float16"), (3, 8, 2, 513, 128, "float16"), (3, 8, 2, 4097, 128, "bfloat16"),
-    (2, 16, 2, 513, 64, "bfloat16"), (2, 16, 2, 1025, 128, "float16"),
+    (2, 16, 2, 1025, 128, "float16"), (2, 16, 1, 513, 64, "bfloat16"), (2, 16, 1, 1025, 128, "float16"),
     (3, 4, 1, 8193, 96, "float16"), (3, 4, 2, 129, 256, "bfloat16"), (2, 2, 2, 1025, 256, "float16"),
     (2, 16, 1, 8193, 512, "float16"), (2, 2, 1, 32769, 256, "float16"), (32, 8, 8, 7200, 64, "bfloat16"),
     (3, 8, 2, 65, 128, "bfloat16"), (2, 4, 4, 3, 128, "float16")])
@@ -39,13 +39,13 @@ def test_lengths_on_both_sides_of_the_lines(B, Hq, Hkv, L, D, dtype_name):
 
 
 @pytest.mark.parametrize("dtype_name", ["float16", "bfloat16"])
-@pytest.mark.parametrize("B,Hkv,L", [(2, 8, 700), (4, 8, 5000), (17, 8, 4100), (2, 2, 257), (2, 2, 1025), (2, 2, 2049),
+@pytest.mark.parametrize("B,Hkv,L", [(2, 8, 700), (4, 8, 5000), (17, 8, 4100), (2, 2, 65), (2, 1, 257), (2, 2, 1025), (2, 2, 2049),
                                      (2, 1, 32769)])
 def test_8bit_lengths(B, Hkv, L, dtype_name):
     import torch
     from gmlx_amd import ops
     rng = np.random.default_rng(L)
-    D, Hq = 64, 2 * Hkv
+    D, Hq = 64, (16 if L == 257 else 2) * Hkv  # (one split up to 256 past eight query heads a kv head)
     q, k, v = _rows(rng, torch, B, Hq, Hkv, L, D, getattr(torch, dtype_name))
     kw, ks, kb, kd = q8_affine(k.float().numpy(), dtype_name)
     vw, vs, vb, vd = q8_affine(v.float().numpy(), dtype_name)
