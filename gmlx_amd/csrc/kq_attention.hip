@@ -1397,7 +1397,8 @@ extern "C" int kq_sdpa_decode_gqa_noalloc(const void *q, const void *k, const vo
                                           kq_stream_t stream) {
     if (B == 0) return KQ_OK;
     if (B < 0 || Hq <= 0 || Hkv <= 0 || Hq % Hkv || D <= 0 || L < 0) return KQ_ERR_BAD_SHAPE;
-    if (ws_layout(B, Hq, Hkv, D, L, false, true).bytes() > KQ_SDPA_NOALLOC_SCRATCH_BYTES) return KQ_ERR_WORKSPACE_TOO_SMALL;
+    const WsLayout least = ws_layout(B, Hq, Hkv, D, L, false, true);
+    if (least.bytes() > KQ_SDPA_NOALLOC_SCRATCH_BYTES) return KQ_ERR_WORKSPACE_TOO_SMALL;
     void *ws = nullptr;
     if (const int rc = scratch_ptr(&ws)) return rc;
     const PaddedKv pad{batch_stride, head_stride, starts};

@@ -2578,7 +2578,8 @@ int kq_stream_launch(const kq_matmul_problem *ps, int n, const int32_t *x_exp, i
 // Streaming expert gather (see kq_sgather_kernel).  Forms: K of 2, 3, 4, 6, 8
 // or 12 super-blocks (16 and 28 for IQ2_XXS), at most 1024 experts, one
 // expert's matrix below 2^31 bytes.  Routing (measured at the C4 / C5
-// layers): the K-quant GLU gathers come here (C4 gate|up 61 us against 67
+// layers) of what the matrix-core tiles leave (kq_gemm_gather_eligible): the
+// K-quant GLU gathers come here (C4 gate|up 61 us against 67
 // for the per-tile kernels); the per-pair down gathers (C4 67 against 65) and
 // the IQ2_XXS gathers (C5 256 / 116 against 165 / 88) stay on the per-tile
 // kernels.  GMLX_KQ_SGATHER=0 declines every call, =2 takes every form.
